@@ -11,8 +11,11 @@
 //    (lane-owned columns), folds its waves together through LDS in a fixed
 //    tree order and writes one fp32 partial row; a second kernel sums the
 //    partial rows in fixed order. No atomics, bit-reproducible run to run.
-//  * generic path (any width, stride or alignment): one 256-thread block per
-//    row with scalar accesses.
+//  * block path (rows too wide for one wave, and any width or alignment with
+//    one element per access): the waves of a block share a row, each thread
+//    holding its columns in registers, so a row is still read once.
+//  * generic path (wider still): one 256-thread block per row, scalar
+//    accesses, the row read again in each pass.
 //  * residual form (Qwen3's `h = residual + attn_out; post_attention_layernorm(h)`):
 //    the forward reads x and the residual, stores s = x + residual rounded
 //    to x's dtype (what the separate add produces) and normalises that s;
@@ -37,10 +40,16 @@ constexpr int kFwdWaves = 4;        // rows per forward block (one wave per row)
 constexpr int kBwdWaves = 8;        // waves per backward block
 constexpr int kMaxBwdBlocks = 256;  // dW partial rows (one 8-wave block per CU)
 constexpr int kGenericThreads = 256;
+constexpr int kBlockThreads = 512;  // most threads that share a row on the block path
 
 // Column of chunk `it` for `lane`, clamped to the last valid chunk of the row.
 __device__ __forceinline__ int clamp_col(int it, int lane, int cols, int vec) {
   const int c = (it * 64 + lane) * vec;
+  return c < cols ? c : cols - vec;
+}
+
+__device__ __forceinline__ int clamp_chunk(int chunk, int cols, int vec) {
+  const int c = chunk * vec;
   return c < cols ? c : cols - vec;
 }
 
@@ -55,12 +64,12 @@ __device__ __forceinline__ float block_sum_256(float v, float* red /* [4] */) {
 
 // ------------------------------------------------------------ fast forward
 // ADD: x <- round(x + res) first (stored to sum), as the residual form does.
-template <typename TX, typename TW, int ITERS, bool ADD>
+// VEC: elements per access, 16 bytes' worth or 1 (odd widths and strides).
+template <typename TX, typename TW, int VEC, int ITERS, bool ADD>
 __global__ __launch_bounds__(64 * kFwdWaves) void rms_fwd_reg(
     const TX* __restrict__ x, int64_t ldx, const TX* __restrict__ res, int64_t ldr,
     TX* __restrict__ sum, int64_t lds, const TW* __restrict__ w, TX* __restrict__ y, int64_t ldy,
     float* __restrict__ rrms, int64_t rows, int cols, float eps) {
-  constexpr int VEC = vec16<TX>();
   const int lane = threadIdx.x & 63;
   const int64_t row = (int64_t)blockIdx.x * kFwdWaves + (threadIdx.x >> 6);
   if (row >= rows) return;
@@ -115,6 +124,61 @@ __global__ __launch_bounds__(64 * kFwdWaves) void rms_fwd_reg(
   }
 }
 
+// ----------------------------------------------------------- block forward
+// One row per block: thread t holds chunks t, t + T, ... (VEC elements each)
+// and the sum of squares crosses the block's waves through LDS. A row is read
+// once where the generic kernel reads it twice with 2- or 4-byte accesses.
+template <typename TX, typename TW, int VEC, int ITERS, bool ADD>
+__global__ __launch_bounds__(kBlockThreads) void rms_fwd_block(
+    const TX* __restrict__ x, int64_t ldx, const TX* __restrict__ res, int64_t ldr,
+    TX* __restrict__ sum, int64_t lds, const TW* __restrict__ w, TX* __restrict__ y, int64_t ldy,
+    float* __restrict__ rrms, int cols, float eps) {
+  __shared__ float red[kBlockThreads / 64];
+  const int T = blockDim.x;
+  const int64_t row = blockIdx.x;
+  const TX* xr = x + row * ldx;
+  float v[ITERS][VEC], rv[ADD ? ITERS : 1][VEC];
+#pragma unroll
+  for (int it = 0; it < ITERS; ++it) {
+    const int c = clamp_chunk(it * T + threadIdx.x, cols, VEC);
+    load_n_nt<TX, VEC>(xr + c, v[it]);
+    if constexpr (ADD) load_n_nt<TX, VEC>(res + row * ldr + c, rv[it]);
+  }
+  float ss = 0.f;
+#pragma unroll
+  for (int it = 0; it < ITERS; ++it) {
+    const int c = (it * T + (int)threadIdx.x) * VEC;
+    if constexpr (ADD) {
+#pragma unroll
+      for (int e = 0; e < VEC; ++e) v[it][e] = to_f32(from_f32<TX>(v[it][e] + rv[it][e]));
+      if (c < cols) store_n_nt<TX, VEC>(sum + row * lds + c, v[it]);
+    }
+    if (c < cols) {
+#pragma unroll
+      for (int e = 0; e < VEC; ++e) ss += v[it][e] * v[it][e];
+    }
+  }
+  ss = wave_sum(ss);
+  if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = ss;
+  __syncthreads();
+  ss = 0.f;
+  for (int i = 0; i < T / 64; ++i) ss += red[i];
+  const float r = 1.0f / sqrtf(ss / (float)cols + eps);
+  if (rrms != nullptr && threadIdx.x == 0) rrms[row] = r;
+  TX* yr = y + row * ldy;
+#pragma unroll
+  for (int it = 0; it < ITERS; ++it) {
+    const int c = (it * T + (int)threadIdx.x) * VEC;
+    if (c < cols) {
+      float wv[VEC], o[VEC];
+      load_n<TW, VEC>(w + c, wv);
+#pragma unroll
+      for (int e = 0; e < VEC; ++e) o[e] = (v[it][e] * r) * wv[e];
+      store_n_nt<TX, VEC>(yr + c, o);
+    }
+  }
+}
+
 // --------------------------------------------------------- generic forward
 // res == nullptr: plain norm of x. Otherwise each thread stores
 // round(x + res) for its columns and normalises that.
@@ -147,13 +211,12 @@ __global__ __launch_bounds__(kGenericThreads) void rms_fwd_generic(
 
 // ------------------------------------------------------------ fast backward
 // HAS_DRES: dx += dres (the residual form's second gradient) before rounding.
-template <typename TX, typename TW, int ITERS, bool HAS_RRMS, bool HAS_DRES>
+template <typename TX, typename TW, int VEC, int ITERS, bool HAS_RRMS, bool HAS_DRES>
 __global__ __launch_bounds__(64 * kBwdWaves) void rms_bwd_reg(
     const TX* __restrict__ x, int64_t ldx, const TW* __restrict__ w, const TX* __restrict__ dy,
     int64_t lddy, const TX* __restrict__ dres, int64_t ldd, const float* __restrict__ rrms,
     float eps, TX* __restrict__ dx, int64_t lddx, float* __restrict__ partial, int64_t rows,
     int cols) {
-  constexpr int VEC = vec16<TX>();
   extern __shared__ float smem[];  // [kBwdWaves/2][cols]
   const int lane = threadIdx.x & 63;
   const int wave = threadIdx.x >> 6;
@@ -283,6 +346,124 @@ __global__ __launch_bounds__(64 * kBwdWaves) void rms_bwd_reg(
   }
 }
 
+// ---------------------------------------------------------- block backward
+// Bound by HBM. A block walks rows b, b + G, ... in batches of R; its threads
+// share each row (thread t: chunks t, t + T, ...), so the per-column dW sums
+// stay in the owning thread's registers and leave as the block's partial row
+// with no fold between waves. Per batch one barrier: the R dot products cross
+// the waves through LDS (two buffers, so the next batch's writes need no
+// second barrier) while the next batch's loads are in flight.
+template <typename TX, typename TW, int VEC, int ITERS, int R, bool HAS_RRMS, bool HAS_DRES>
+__global__ __launch_bounds__(kBlockThreads) void rms_bwd_block(
+    const TX* __restrict__ x, int64_t ldx, const TW* __restrict__ w, const TX* __restrict__ dy,
+    int64_t lddy, const TX* __restrict__ dres, int64_t ldd, const float* __restrict__ rrms,
+    float eps, TX* __restrict__ dx, int64_t lddx, float* __restrict__ partial, int64_t rows,
+    int cols) {
+  constexpr int kWaves = kBlockThreads / 64;
+  constexpr int kVals = HAS_RRMS ? 1 : 2;  // g w . x, and x . x when rrms is not given
+  __shared__ float red[2][kVals][R][kWaves];
+  const int T = blockDim.x;
+  const int nw = T >> 6;
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  using P = Pack<TX, VEC>;
+  struct Batch {
+    P x[R][ITERS], g[R][ITERS], d[HAS_DRES ? R : 1][HAS_DRES ? ITERS : 1];
+    float r[R];
+  };
+
+  float wv[ITERS][VEC], acc[ITERS][VEC];
+#pragma unroll
+  for (int it = 0; it < ITERS; ++it) {
+    load_n<TW, VEC>(w + clamp_chunk(it * T + threadIdx.x, cols, VEC), wv[it]);
+#pragma unroll
+    for (int e = 0; e < VEC; ++e) acc[it][e] = 0.f;
+  }
+  // rows past the end load the last row, chunks past the end the last chunk;
+  // neither is used
+  auto load = [&](Batch& b, int64_t first) {
+#pragma unroll
+    for (int k = 0; k < R; ++k) {
+      int64_t row = first + (int64_t)k * gridDim.x;
+      row = row < rows ? row : rows - 1;
+#pragma unroll
+      for (int it = 0; it < ITERS; ++it) {
+        const int c = clamp_chunk(it * T + threadIdx.x, cols, VEC);
+        b.x[k][it] = load_pack_nt<TX, VEC>(x + row * ldx + c);
+        b.g[k][it] = load_pack_nt<TX, VEC>(dy + row * lddy + c);
+        if constexpr (HAS_DRES) b.d[k][it] = load_pack_nt<TX, VEC>(dres + row * ldd + c);
+      }
+      if constexpr (HAS_RRMS) b.r[k] = rrms[row];
+    }
+  };
+
+  const int64_t step = (int64_t)gridDim.x * R;
+  Batch cur, next;
+  load(cur, blockIdx.x);
+  int buf = 0;
+  for (int64_t first = blockIdx.x; first < rows; first += step, buf ^= 1) {
+#pragma unroll
+    for (int k = 0; k < R; ++k) {
+      float dot = 0.f, ss = 0.f;
+#pragma unroll
+      for (int it = 0; it < ITERS; ++it) {
+        if ((it * T + (int)threadIdx.x) * VEC < cols) {
+#pragma unroll
+          for (int e = 0; e < VEC; ++e) {
+            const float xv = to_f32(cur.x[k][it].v[e]);
+            dot += (to_f32(cur.g[k][it].v[e]) * wv[it][e]) * xv;
+            if constexpr (!HAS_RRMS) ss += xv * xv;
+          }
+        }
+      }
+      dot = wave_sum(dot);
+      if constexpr (!HAS_RRMS) ss = wave_sum(ss);
+      if (lane == 0) {
+        red[buf][0][k][wave] = dot;
+        if constexpr (!HAS_RRMS) red[buf][kVals - 1][k][wave] = ss;
+      }
+    }
+    if (first + step < rows) load(next, first + step);
+    __syncthreads();
+#pragma unroll
+    for (int k = 0; k < R; ++k) {
+      const int64_t row = first + (int64_t)k * gridDim.x;
+      if (row >= rows) break;
+      float dot = 0.f, r;
+      for (int i = 0; i < nw; ++i) dot += red[buf][0][k][i];
+      if constexpr (HAS_RRMS) {
+        r = cur.r[k];
+      } else {
+        float ss = 0.f;
+        for (int i = 0; i < nw; ++i) ss += red[buf][kVals - 1][k][i];
+        r = 1.0f / sqrtf(ss / (float)cols + eps);
+      }
+      const float mean = dot / (float)cols;
+      const float r3 = (r * r) * r;
+#pragma unroll
+      for (int it = 0; it < ITERS; ++it) {
+        const int c = (it * T + (int)threadIdx.x) * VEC;
+        if (c >= cols) continue;
+        float o[VEC];
+#pragma unroll
+        for (int e = 0; e < VEC; ++e) {
+          const float xv = to_f32(cur.x[k][it].v[e]), gv = to_f32(cur.g[k][it].v[e]);
+          o[e] = (gv * wv[it][e]) * r - (xv * mean) * r3;
+          if constexpr (HAS_DRES) o[e] = o[e] + to_f32(cur.d[k][it].v[e]);
+          acc[it][e] += gv * (xv * r);
+        }
+        store_n_nt<TX, VEC>(dx + row * lddx + c, o);
+      }
+    }
+    cur = next;
+  }
+  float* pr = partial + (int64_t)blockIdx.x * cols;
+#pragma unroll
+  for (int it = 0; it < ITERS; ++it) {
+    const int c = (it * T + (int)threadIdx.x) * VEC;
+    if (c < cols) store_n<float, VEC>(pr + c, acc[it]);
+  }
+}
+
 // --------------------------------------------------------- generic backward
 // Block b handles rows b, b+G, ...; thread t owns columns t, t+256, ... of
 // partial row b (so no two threads touch the same partial element).
@@ -383,15 +564,45 @@ __global__ __launch_bounds__(256) void rms_dw_reduce(const float* __restrict__ p
   }
 }
 
-// Register-path capacity: ITERS chunks of 16 bytes per lane. The backward
-// holds three row-sized arrays per lane, so it stops at 32 values per array.
-template <typename TX>
-int pick_iters(int64_t cols, bool backward) {
-  const int64_t per = 64 * vec16<TX>();
-  const int max_it = backward ? 32 / vec16<TX>() : 8;
+// Rows a block-path backward holds at once, with as many in flight behind
+// them: 4 chunks per thread and operand in 16-byte vectors (16 VGPRs; twice
+// as many spill with a residual gradient), 16 single elements.
+constexpr int batch_rows(int vec, int iters) {
+  const int r = (vec == 1 ? 16 : 4) / iters;
+  return r < 1 ? 1 : r > 4 ? 4 : r;
+}
+
+// How a call of `cols` columns runs, from the widest access that its widths,
+// strides and bases allow (vec: 16 bytes' worth of elements, or 1):
+//   kWave   one wave per row, iters chunks per lane. The forward holds one
+//           row per lane and takes up to 8 chunks; the backward holds three
+//           row-sized fp32 arrays, so it stops at 32 values per array.
+//   kBlock  rows wider than that: a block of `threads` per row, the fewest
+//           chunks per thread that keep it within kBlockThreads.
+//   kScalar wider still (over 8192 columns one element at a time, 16384 in
+//           16-bit or 8192 in fp32 vectors): the generic kernels.
+// Measured with a residual: bf16 [3333, 4096] backward 209 us generic, 27 us
+// block (4.0 TB/s); fp32 [8192, 5120] forward 191 -> 115 us, backward 856 ->
+// 115 us (5.8 TB/s); bf16 [8192, 5119] 159 -> 72 and 800 -> 85 us; without,
+// bf16 [8192, 301] (one element per access, a wave per row) 12.1 -> 6.4 and
+// 39 -> 9 us. At 2048 columns the wave path is the faster one (backward,
+// fp32 42 against 46 us, bf16 with a residual 29 against 38).
+enum class Path { kWave, kBlock, kScalar };
+struct Plan {
+  Path path;
+  int iters, threads;
+};
+
+Plan pick_plan(int64_t cols, int vec, bool backward) {
+  const int64_t chunks = (cols + vec - 1) / vec;
+  const int max_wave = backward && 32 / vec < 8 ? 32 / vec : 8;
   for (int it : {1, 2, 4, 8})
-    if (it <= max_it && cols <= per * it) return it;
-  return 0;
+    if (it <= max_wave && chunks <= 64 * it) return {Path::kWave, it, 64};
+  const int max_block = vec == 1 ? 16 : 4;
+  for (int it = 1; it <= max_block; it *= 2)
+    if (chunks <= (int64_t)kBlockThreads * it)
+      return {Path::kBlock, it, (int)(((chunks + it - 1) / it + 63) / 64 * 64)};
+  return {Path::kScalar, 0, 0};
 }
 
 // A row operand: base pointer and row stride in elements (ptr may be null:
@@ -401,11 +612,10 @@ struct RowOp {
   int64_t ld;
 };
 
-template <typename TX, typename TW>
-bool fast_path_ok(bool backward, const void* w, int64_t cols, std::initializer_list<RowOp> ops) {
-  constexpr int VEC = vec16<TX>();
-  if (cols % VEC != 0 || pick_iters<TX>(cols, backward) == 0) return false;
-  if (!aligned16(w)) return false;
+// Whether every row of every operand can be accessed in 16-byte vectors.
+template <typename TX>
+bool vector_ok(const void* w, int64_t cols, std::initializer_list<RowOp> ops) {
+  if (cols % vec16<TX>() != 0 || !aligned16(w)) return false;
   for (const RowOp& o : ops)
     if (o.ptr != nullptr && (!aligned16(o.ptr) || (o.ld * (int64_t)sizeof(TX)) % 16 != 0))
       return false;
@@ -423,29 +633,64 @@ int launch_fwd(const void* x, int64_t ldx, const void* res, int64_t ldr, void* s
   TX* sp = static_cast<TX*>(sum);
   const TW* wp = static_cast<const TW*>(w);
   TX* yp = static_cast<TX*>(y);
-  if (fast_path_ok<TX, TW>(false, w, cols, {{x, ldx}, {y, ldy}, {res, ldr}, {sum, lds}})) {
+  const bool vec = vector_ok<TX>(w, cols, {{x, ldx}, {y, ldy}, {res, ldr}, {sum, lds}});
+  const Plan plan = pick_plan(cols, vec ? vec16<TX>() : 1, false);
+  if (plan.path == Path::kWave) {
     const dim3 grid((unsigned)((rows + kFwdWaves - 1) / kFwdWaves));
-    const int it = pick_iters<TX>(cols, false);
-#define ML_FWD(I, A)                                                                         \
-  rms_fwd_reg<TX, TW, I, A><<<grid, 64 * kFwdWaves, 0, st>>>(xp, ldx, rp, ldr, sp, lds, wp, yp, \
-                                                             ldy, rrms, rows, (int)cols, eps)
-#define ML_FWD_A(I)  \
-  if (rp) {          \
-    ML_FWD(I, true); \
-  } else {           \
-    ML_FWD(I, false); \
+#define ML_FWD(V, I, A)                                                                          \
+  rms_fwd_reg<TX, TW, V, I, A><<<grid, 64 * kFwdWaves, 0, st>>>(xp, ldx, rp, ldr, sp, lds, wp,   \
+                                                                yp, ldy, rrms, rows, (int)cols, eps)
+#define ML_FWD_I(V, A)              \
+  switch (plan.iters) {             \
+    case 1: ML_FWD(V, 1, A); break; \
+    case 2: ML_FWD(V, 2, A); break; \
+    case 4: ML_FWD(V, 4, A); break; \
+    default: ML_FWD(V, 8, A); break; \
   }
-    switch (it) {
-      case 1: ML_FWD_A(1); break;
-      case 2: ML_FWD_A(2); break;
-      case 4: ML_FWD_A(4); break;
-      default: ML_FWD_A(8); break;
+    if (vec && rp) {
+      ML_FWD_I(vec16<TX>(), true);
+    } else if (vec) {
+      ML_FWD_I(vec16<TX>(), false);
+    } else if (rp) {
+      ML_FWD_I(1, true);
+    } else {
+      ML_FWD_I(1, false);
+    }
+#undef ML_FWD_I
+#undef ML_FWD
+    ML_LAUNCH_CHECK();
+    return ML_OK;
+  }
+  ML_CHECK(rows <= 0x7fffffffLL, "rmsnorm: too many rows for a block per row (%lld)",
+           (long long)rows);
+  if (plan.path == Path::kBlock) {
+#define ML_FWD(V, I, A)                                                                      \
+  rms_fwd_block<TX, TW, V, I, A><<<dim3((unsigned)rows), plan.threads, 0, st>>>(             \
+      xp, ldx, rp, ldr, sp, lds, wp, yp, ldy, rrms, (int)cols, eps)
+#define ML_FWD_A(V, I)  \
+  if (rp) {             \
+    ML_FWD(V, I, true); \
+  } else {              \
+    ML_FWD(V, I, false); \
+  }
+    if (vec) {
+      constexpr int V = vec16<TX>();
+      if (plan.iters <= 2) {  // 1 chunk per thread: always within the wave path
+        ML_FWD_A(V, 2);
+      } else {
+        ML_FWD_A(V, 4);
+      }
+    } else {
+      switch (plan.iters) {
+        case 2: ML_FWD_A(1, 2); break;
+        case 4: ML_FWD_A(1, 4); break;
+        case 8: ML_FWD_A(1, 8); break;
+        default: ML_FWD_A(1, 16); break;
+      }
     }
 #undef ML_FWD_A
 #undef ML_FWD
   } else {
-    ML_CHECK(rows <= 0x7fffffffLL, "rmsnorm: too many rows for the generic path (%lld)",
-             (long long)rows);
     rms_fwd_generic<TX, TW><<<dim3((unsigned)rows), kGenericThreads, 0, st>>>(
         xp, ldx, rp, ldr, sp, lds, wp, yp, ldy, rrms, rows, cols, eps);
   }
@@ -453,11 +698,13 @@ int launch_fwd(const void* x, int64_t ldx, const void* res, int64_t ldr, void* s
   return ML_OK;
 }
 
-int64_t bwd_blocks_fast(int64_t rows) {
+// dW partial rows: one per block. The wave path's blocks take kBwdWaves rows
+// at a time, the others' one batch or row each.
+int64_t bwd_blocks_wave(int64_t rows) {
   const int64_t b = (rows + kBwdWaves - 1) / kBwdWaves;
   return b < kMaxBwdBlocks ? b : kMaxBwdBlocks;
 }
-int64_t bwd_blocks_generic(int64_t rows) { return rows < kMaxBwdBlocks ? rows : kMaxBwdBlocks; }
+int64_t bwd_blocks_row(int64_t rows) { return rows < kMaxBwdBlocks ? rows : kMaxBwdBlocks; }
 
 // dres: the residual form's second gradient of the sum (null: plain norm).
 template <typename TX, typename TW>
@@ -472,42 +719,75 @@ int launch_bwd(const void* x, int64_t ldx, const void* w, const void* dy, int64_
   TX* dxp = static_cast<TX*>(dx);
   TW* dwp = static_cast<TW*>(dw);
   float* part = static_cast<float*>(ws);
-  const int64_t lds_bytes = (int64_t)(kBwdWaves / 2) * cols * (int64_t)sizeof(float);
-  const bool fast =
-      fast_path_ok<TX, TW>(true, w, cols, {{x, ldx}, {dx, lddx}, {dy, lddy}, {dres, ldd}}) &&
-      lds_bytes <= 64 * 1024;
-  const int64_t G = rows == 0 ? 0 : (fast ? bwd_blocks_fast(rows) : bwd_blocks_generic(rows));
+  const bool vec = vector_ok<TX>(w, cols, {{x, ldx}, {dx, lddx}, {dy, lddy}, {dres, ldd}});
+  const Plan plan = pick_plan(cols, vec ? vec16<TX>() : 1, true);
+  const int64_t G = plan.path == Path::kWave ? bwd_blocks_wave(rows) : bwd_blocks_row(rows);
   ML_CHECK(ws_bytes >= (size_t)(G * cols * (int64_t)sizeof(float)),
            "rmsnorm backward: workspace too small (%zu < %lld bytes)", ws_bytes,
            (long long)(G * cols * (int64_t)sizeof(float)));
   if (G > 0) {
-    if (fast) {
-      const int it = pick_iters<TX>(cols, true);
-#define ML_BWD(I, R, D)                                                                           \
-  rms_bwd_reg<TX, TW, I, R, D><<<dim3((unsigned)G), 64 * kBwdWaves, (size_t)lds_bytes, st>>>( \
-      xp, ldx, wp, gp, lddy, dp, ldd, rrms, eps, dxp, lddx, part, rows, (int)cols)
-#define ML_BWD_R(I)          \
-  if (rrms && dp) {          \
-    ML_BWD(I, true, true);   \
-  } else if (rrms) {         \
-    ML_BWD(I, true, false);  \
-  } else if (dp) {           \
-    ML_BWD(I, false, true);  \
-  } else {                   \
-    ML_BWD(I, false, false); \
+    // the fold of the waves' dW sums: at most 2048 columns, 32 KB
+    const int lds_bytes = (int)((kBwdWaves / 2) * cols * (int64_t)sizeof(float));
+#define ML_BWD_R(V, I)          \
+  if (rrms && dp) {             \
+    ML_BWD(V, I, true, true);   \
+  } else if (rrms) {            \
+    ML_BWD(V, I, true, false);  \
+  } else if (dp) {              \
+    ML_BWD(V, I, false, true);  \
+  } else {                      \
+    ML_BWD(V, I, false, false); \
   }
-      switch (it) {
-        case 1: ML_BWD_R(1); break;
-        case 2: ML_BWD_R(2); break;
-        case 4: ML_BWD_R(4); break;
-        default:
-          if constexpr (vec16<TX>() * 8 <= 32) {
-            ML_BWD_R(8);
-          }
-          break;
+    constexpr int V = vec16<TX>();
+    if (plan.path == Path::kWave) {
+#define ML_BWD(VEC, I, R, D)                                                               \
+  rms_bwd_reg<TX, TW, VEC, I, R, D><<<dim3((unsigned)G), 64 * kBwdWaves, lds_bytes, st>>>( \
+      xp, ldx, wp, gp, lddy, dp, ldd, rrms, eps, dxp, lddx, part, rows, (int)cols)
+      if (vec) {
+        switch (plan.iters) {
+          case 1: ML_BWD_R(V, 1); break;
+          case 2: ML_BWD_R(V, 2); break;
+          case 4: ML_BWD_R(V, 4); break;
+          default:
+            if constexpr (V * 8 <= 32) {
+              ML_BWD_R(V, 8);
+            }
+            break;
+        }
+      } else {
+        switch (plan.iters) {
+          case 1: ML_BWD_R(1, 1); break;
+          case 2: ML_BWD_R(1, 2); break;
+          case 4: ML_BWD_R(1, 4); break;
+          default: ML_BWD_R(1, 8); break;
+        }
       }
-#undef ML_BWD_R
 #undef ML_BWD
+    } else if (plan.path == Path::kBlock) {
+#define ML_BWD(VEC, I, R, D)                                                                      \
+  rms_bwd_block<TX, TW, VEC, I, batch_rows(VEC, I), R, D>                                         \
+      <<<dim3((unsigned)G), plan.threads, 0, st>>>(xp, ldx, wp, gp, lddy, dp, ldd, rrms, eps, dxp, \
+                                                   lddx, part, rows, (int)cols)
+      if (vec) {
+        switch (plan.iters) {
+          case 1:
+            if constexpr (V * 512 > 2048) {  // fp32: within the wave path
+              ML_BWD_R(V, 1);
+            }
+            break;
+          case 2: ML_BWD_R(V, 2); break;
+          default: ML_BWD_R(V, 4); break;
+        }
+      } else {
+        switch (plan.iters) {
+          case 2: ML_BWD_R(1, 2); break;
+          case 4: ML_BWD_R(1, 4); break;
+          case 8: ML_BWD_R(1, 8); break;
+          default: ML_BWD_R(1, 16); break;
+        }
+      }
+#undef ML_BWD
+#undef ML_BWD_R
     } else {
       if (rrms)
         rms_bwd_generic<TX, TW, true><<<dim3((unsigned)G), kGenericThreads, 0, st>>>(
@@ -585,7 +865,7 @@ extern "C" int ml_rmsnorm_add_fwd(const void* x, int64_t ldx, const void* residu
 
 extern "C" size_t ml_rmsnorm_bwd_workspace_bytes(int64_t rows, int64_t cols) {
   if (rows <= 0 || cols <= 0) return 0;
-  const int64_t g = bwd_blocks_generic(rows);  // >= the fast path's block count
+  const int64_t g = bwd_blocks_row(rows);  // >= the wave path's block count
   return (size_t)(g * cols * (int64_t)sizeof(float));
 }
 
