@@ -31,7 +31,7 @@
 extern "C" {
 #endif
 
-#define ML_ABI_VERSION 6
+#define ML_ABI_VERSION 7
 
 /* dtype tags */
 #define ML_F32 0
@@ -477,6 +477,20 @@ int ml_gemm_f32_segments(int64_t M, int64_t N, int nseg, const int64_t* k_lens,
                          const void* const* b_ptrs, const int64_t* ldbs, int a_layout,
                          int b_layout, float* C, int64_t ldc, float alpha, float beta,
                          void* stream);
+
+/*
+ * ml_gemm_f32_segments with a workspace for the partial sums of a product
+ * whose output tiles alone would not fill the GPU: K (the sum of k_lens) is
+ * then split over workgroups and the partials summed in a fixed order. The
+ * query returns what such a split of [M, K] x [K, N] takes (0: not split); a
+ * null or smaller workspace means no split.
+ */
+size_t ml_gemm_f32_workspace_bytes(int64_t M, int64_t N, int64_t K);
+int ml_gemm_f32_segments_ws(int64_t M, int64_t N, int nseg, const int64_t* k_lens,
+                            const void* const* a_ptrs, const int64_t* ldas,
+                            const void* const* b_ptrs, const int64_t* ldbs, int a_layout,
+                            int b_layout, float* C, int64_t ldc, float alpha, float beta,
+                            void* workspace, size_t workspace_bytes, void* stream);
 
 #ifdef __cplusplus
 }

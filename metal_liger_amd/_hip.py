@@ -108,6 +108,12 @@ SIGNATURES: dict[str, tuple] = {
         [_i64, _i64, _i32, _i64p, ctypes.POINTER(_p), _i64p, ctypes.POINTER(_p), _i64p, _i32, _i32,
          _p, _i64, _f32, _f32, _p],
     ),
+    "ml_gemm_f32_workspace_bytes": (_sz, [_i64, _i64, _i64]),
+    "ml_gemm_f32_segments_ws": (
+        _i32,
+        [_i64, _i64, _i32, _i64p, ctypes.POINTER(_p), _i64p, ctypes.POINTER(_p), _i64p, _i32, _i32,
+         _p, _i64, _f32, _f32, _p, _sz, _p],
+    ),
     "ml_flce_fwd_grad_f32_workspace_bytes": (_sz, [_i64, _i64, _i64]),
     "ml_flce_fwd_grad_f32": (
         _i32,
@@ -139,7 +145,7 @@ SIGNATURES: dict[str, tuple] = {
     ),
 }
 
-ABI_VERSION = 6
+ABI_VERSION = 7
 
 _lib = None
 _lock = threading.Lock()

@@ -568,11 +568,14 @@ def gemm_f32(a_list, b_list, a_t: bool = False, b_t: bool = False, alpha: float 
         return out
     if sum(ks) == 0:
         return out.zero_()
+    ws_bytes = _hip.query("ml_gemm_f32_workspace_bytes", M, N, sum(ks))
+    ws = torch.empty(ws_bytes // 4, dtype=torch.float32, device=out.device) if ws_bytes else None
     call(
-        "ml_gemm_f32_segments", M, N, len(ks), geom(ks), _hip.ptrs([a.data_ptr() for a in a_list]),
-        geom([a.stride(0) for a in a_list]), _hip.ptrs([b.data_ptr() for b in b_list]),
-        geom([b.stride(0) for b in b_list]), 1 if a_t else 0, 0 if b_t else 1, ptr(out),
-        out.stride(0), float(alpha), 0.0, stream_of(a_list[0]),
+        "ml_gemm_f32_segments_ws", M, N, len(ks), geom(ks),
+        _hip.ptrs([a.data_ptr() for a in a_list]), geom([a.stride(0) for a in a_list]),
+        _hip.ptrs([b.data_ptr() for b in b_list]), geom([b.stride(0) for b in b_list]),
+        1 if a_t else 0, 0 if b_t else 1, ptr(out), out.stride(0), float(alpha), 0.0, ptr(ws),
+        ws_bytes, stream_of(a_list[0]),
     )
     return out
 
