@@ -31,7 +31,7 @@
 extern "C" {
 #endif
 
-#define ML_ABI_VERSION 7
+#define ML_ABI_VERSION 8
 
 /* dtype tags */
 #define ML_F32 0
@@ -438,6 +438,18 @@ int ml_gemm_bf16_segments(int64_t M, int64_t N, int nseg, const int64_t* k_lens,
                           const int64_t* ldbs, int a_layout, int b_layout, void* C, int64_t ldc,
                           int c_dtype, float alpha, float beta, void* stream);
 
+/* ml_gemm_bf16_segments with a workspace for the fp32 partial sums of a
+ * product whose output tiles alone would not fill the GPU (a_layout 0): the
+ * k-tiles of all segments are then split over workgroups and the partials
+ * summed in a fixed order. The query returns what such a split takes (0: K is
+ * not split); a null or smaller workspace means no split. */
+size_t ml_gemm_bf16_segments_workspace_bytes(int64_t M, int64_t N, int nseg, const int64_t* k_lens);
+int ml_gemm_bf16_segments_ws(int64_t M, int64_t N, int nseg, const int64_t* k_lens,
+                             const void* const* a_ptrs, const int64_t* ldas,
+                             const void* const* b_ptrs, const int64_t* ldbs, int a_layout,
+                             int b_layout, void* C, int64_t ldc, int c_dtype, float alpha,
+                             float beta, void* workspace, size_t workspace_bytes, void* stream);
+
 /* count (1..3) independent segmented products in ONE launch, A [M_g, K]
  * row-major (a_layout 0) for every product: product g has nseg[g] segments,
  * the next nseg[g] entries of k_lens / a_ptrs / ldas / b_ptrs / ldbs, and
@@ -454,7 +466,8 @@ int ml_gemm_bf16_segments_group(int count, const int64_t* M, const int64_t* N, c
                                 void* stream);
 
 /* Split-K form with a tile shape (tile_cfg 0: 256x256, 1: 256x32 for
- * rank-r outputs, 2: 64x256 for few-row outputs): ksplit slices of K write
+ * rank-r outputs, 2: 64x256 for few-row outputs, 3: 128x128 and 4: 256x256
+ * for a_layout 0, which store C directly when ksplit is 1): ksplit slices of K write
  * fp32 partials to `workspace` (ml_gemm_splitk_workspace_bytes), summed in a
  * fixed order into C = alpha * A B + beta * C. Same operand rules as above. */
 size_t ml_gemm_splitk_workspace_bytes(int64_t M, int64_t N, int64_t K, int ksplit);

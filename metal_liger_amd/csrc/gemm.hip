@@ -8,7 +8,7 @@ namespace gemm {
 namespace {
 
 int run(int64_t M, int64_t N, int nseg, const Segment* segs, int la, int lb, void* C, int64_t ldc,
-        int c_dtype, float alpha, float beta, void* stream) {
+        int c_dtype, float alpha, float beta, void* ws, size_t ws_bytes, void* stream) {
   ML_CHECK(M > 0 && N > 0 && M < (1LL << 31) && N < (1LL << 31), "gemm: bad M=%lld N=%lld",
            (long long)M, (long long)N);
   ML_CHECK(la == kKMajor || la == kMNMajor, "gemm: bad A layout %d", la);
@@ -19,15 +19,20 @@ int run(int64_t M, int64_t N, int nseg, const Segment* segs, int la, int lb, voi
   ML_CHECK(c_dtype != ML_BF16 || (ldc % 8 == 0 && aligned16(C)),
            "gemm: a bf16 C needs ldc a multiple of 8 and a 16-byte aligned base (ldc %lld)",
            (long long)ldc);
-  Problem pb;
-  int rc = make_problem<BigCfg>(pb, (int)M, (int)N, nseg, segs, la, lb, 0);
-  if (rc) return rc;
   hipStream_t st = (hipStream_t)stream;
   // r4 is the faster engine when A is K-major, the big engine otherwise
   if (la == kKMajor) {
-    if (c_dtype == ML_F32) return launch_store<float, R4Cfg>(pb, la, lb, C, ldc, alpha, beta, st);
-    if (c_dtype == ML_BF16) return launch_store<bf16, R4Cfg>(pb, la, lb, C, ldc, alpha, beta, st);
+    float* w = static_cast<float*>(ws);
+    if (c_dtype == ML_F32)
+      return run_product((int)M, (int)N, nseg, segs, lb, static_cast<float*>(C), ldc, alpha, beta,
+                         w, ws_bytes, st);
+    if (c_dtype == ML_BF16)
+      return run_product((int)M, (int)N, nseg, segs, lb, static_cast<bf16*>(C), ldc, alpha, beta,
+                         w, ws_bytes, st);
   } else {
+    Problem pb;
+    int rc = make_problem<BigCfg>(pb, (int)M, (int)N, nseg, segs, la, lb, 0);
+    if (rc) return rc;
     if (c_dtype == ML_F32) return launch_store<float>(pb, la, lb, C, ldc, alpha, beta, st);
     if (c_dtype == ML_BF16) return launch_store<bf16>(pb, la, lb, C, ldc, alpha, beta, st);
   }
@@ -63,6 +68,35 @@ int run_splitk(int64_t M, int64_t N, const Segment& seg, int la, int lb, int ksp
   return ML_ERR_INVALID;
 }
 
+// The same for the r4 engine's tiles (A K-major); one split stores C directly.
+template <class C>
+int run_splitk_r4(int64_t M, int64_t N, const Segment& seg, int la, int lb, int ksplit, void* C_,
+                  int64_t ldc, int c_dtype, float alpha, float beta, void* ws, size_t ws_bytes,
+                  hipStream_t st) {
+  ML_CHECK(la == kKMajor, "gemm: this tile takes a K-major A");
+  ML_CHECK(c_dtype == ML_F32 || c_dtype == ML_BF16, "gemm: C dtype %d not supported (fp32 or bf16)",
+           c_dtype);
+  ML_CHECK(c_dtype != ML_BF16 || (ldc % 8 == 0 && aligned16(C_)),
+           "gemm: a bf16 C needs ldc a multiple of 8 and a 16-byte aligned base (ldc %lld)",
+           (long long)ldc);
+  Problem pb;
+  int rc = make_problem<C>(pb, (int)M, (int)N, 1, &seg, la, lb, 0, ksplit);
+  if (rc) return rc;
+  if (pb.ksplit == 1)
+    return c_dtype == ML_F32 ? launch_store<float, C>(pb, la, lb, C_, ldc, alpha, beta, st)
+                             : launch_store<bf16, C>(pb, la, lb, C_, ldc, alpha, beta, st);
+  ML_CHECK(ws && ws_bytes >= splitk_ws_bytes(pb), "gemm: split-K workspace too small (%zu < %zu)",
+           ws_bytes, splitk_ws_bytes(pb));
+  float* w = static_cast<float*>(ws);
+  auto go = [&](auto* out) {
+    using TC = std::remove_pointer_t<decltype(out)>;
+    return lb == kKMajor
+               ? launch_splitk<C, kKMajor, kKMajor, TC>(pb, w, out, ldc, alpha, beta, st)
+               : launch_splitk<C, kKMajor, kMNMajor, TC>(pb, w, out, ldc, alpha, beta, st);
+  };
+  return c_dtype == ML_F32 ? go(static_cast<float*>(C_)) : go(static_cast<bf16*>(C_));
+}
+
 }  // namespace
 }  // namespace gemm
 }  // namespace mla
@@ -74,7 +108,8 @@ extern "C" int ml_gemm_bf16(int64_t M, int64_t N, int64_t K, const void* A, int6
                             int64_t ldc, int c_dtype, float alpha, float beta, void* stream) {
   ML_CHECK(K >= 0 && K < (1LL << 31), "gemm: bad K=%lld", (long long)K);
   gemm::Segment s{{static_cast<const bf16*>(A), lda}, {static_cast<const bf16*>(B), ldb}, (int)K};
-  return gemm::run(M, N, 1, &s, a_layout, b_layout, C, ldc, c_dtype, alpha, beta, stream);
+  return gemm::run(M, N, 1, &s, a_layout, b_layout, C, ldc, c_dtype, alpha, beta, nullptr, 0,
+                   stream);
 }
 
 extern "C" int ml_gemm_bf16_segments(int64_t M, int64_t N, int nseg, const int64_t* k_lens,
@@ -82,6 +117,27 @@ extern "C" int ml_gemm_bf16_segments(int64_t M, int64_t N, int nseg, const int64
                                      const void* const* b_ptrs, const int64_t* ldbs, int a_layout,
                                      int b_layout, void* C, int64_t ldc, int c_dtype, float alpha,
                                      float beta, void* stream) {
+  return ml_gemm_bf16_segments_ws(M, N, nseg, k_lens, a_ptrs, ldas, b_ptrs, ldbs, a_layout,
+                                  b_layout, C, ldc, c_dtype, alpha, beta, nullptr, 0, stream);
+}
+
+extern "C" size_t ml_gemm_bf16_segments_workspace_bytes(int64_t M, int64_t N, int nseg,
+                                                        const int64_t* k_lens) {
+  if (M <= 0 || N <= 0 || M >= (1LL << 31) || N >= (1LL << 31) || !k_lens) return 0;
+  int64_t kt = 0;
+  for (int s = 0; s < nseg; ++s) {
+    if (k_lens[s] < 0 || k_lens[s] >= (1LL << 31)) return 0;
+    kt += (k_lens[s] + gemm::kBK - 1) / gemm::kBK;
+  }
+  return kt < (1LL << 31) ? gemm::product_ws_bytes((int)M, (int)N, (int)kt) : 0;
+}
+
+extern "C" int ml_gemm_bf16_segments_ws(int64_t M, int64_t N, int nseg, const int64_t* k_lens,
+                                        const void* const* a_ptrs, const int64_t* ldas,
+                                        const void* const* b_ptrs, const int64_t* ldbs,
+                                        int a_layout, int b_layout, void* C, int64_t ldc,
+                                        int c_dtype, float alpha, float beta, void* workspace,
+                                        size_t workspace_bytes, void* stream) {
   ML_CHECK(nseg >= 1 && nseg <= gemm::kMaxSeg, "gemm: 1..%d segments supported (got %d)",
            gemm::kMaxSeg, nseg);
   ML_CHECK(k_lens && a_ptrs && ldas && b_ptrs && ldbs, "gemm: null segment arrays");
@@ -91,7 +147,8 @@ extern "C" int ml_gemm_bf16_segments(int64_t M, int64_t N, int nseg, const int64
     segs[s] = gemm::Segment{{static_cast<const bf16*>(a_ptrs[s]), ldas[s]},
                             {static_cast<const bf16*>(b_ptrs[s]), ldbs[s]}, (int)k_lens[s]};
   }
-  return gemm::run(M, N, nseg, segs, a_layout, b_layout, C, ldc, c_dtype, alpha, beta, stream);
+  return gemm::run(M, N, nseg, segs, a_layout, b_layout, C, ldc, c_dtype, alpha, beta, workspace,
+                   workspace_bytes, stream);
 }
 
 extern "C" int ml_gemm_bf16_segments_group(int count, const int64_t* M, const int64_t* N,
@@ -106,6 +163,8 @@ extern "C" int ml_gemm_bf16_segments_group(int count, const int64_t* M, const in
            "gemm group: null argument arrays");
   ML_CHECK(b_layout == gemm::kKMajor || b_layout == gemm::kMNMajor, "gemm group: bad B layout");
   gemm::Problem pbs[gemm::kMaxGroup];
+  gemm::Segment segs[gemm::kMaxGroup][gemm::kMaxSeg];
+  int ms[gemm::kMaxGroup], ns[gemm::kMaxGroup], kts[gemm::kMaxGroup];
   int base = 0;
   for (int g = 0; g < count; ++g) {
     ML_CHECK(M[g] > 0 && N[g] > 0 && M[g] < (1LL << 31) && N[g] < (1LL << 31),
@@ -116,23 +175,35 @@ extern "C" int ml_gemm_bf16_segments_group(int count, const int64_t* M, const in
              "(product %d, ldc %lld)", g, (long long)ldc[g]);
     ML_CHECK(nseg[g] >= 1 && nseg[g] <= gemm::kMaxSeg, "gemm group: 1..%d segments (product %d)",
              gemm::kMaxSeg, g);
-    gemm::Segment segs[gemm::kMaxSeg];
     for (int s = 0; s < nseg[g]; ++s) {
       const int q = base + s;
       ML_CHECK(k_lens[q] >= 0 && k_lens[q] < (1LL << 31), "gemm group: bad K segment %d", q);
-      segs[s] = gemm::Segment{{static_cast<const bf16*>(a_ptrs[q]), ldas[q]},
+      segs[g][s] = gemm::Segment{{static_cast<const bf16*>(a_ptrs[q]), ldas[q]},
                               {static_cast<const bf16*>(b_ptrs[q]), ldbs[q]}, (int)k_lens[q]};
     }
-    const int rc = gemm::make_problem<gemm::R4Cfg>(pbs[g], (int)M[g], (int)N[g], nseg[g], segs,
-                                                   gemm::kKMajor, b_layout, 0);
-    if (rc) return rc;
+    ms[g] = (int)M[g];
+    ns[g] = (int)N[g];
+    kts[g] = gemm::segment_ktiles(nseg[g], segs[g]);
     base += nseg[g];
   }
+  const bool small = gemm::plan_products(count, ms, ns, kts, false).tile == 128;
+  for (int g = 0; g < count; ++g) {
+    const int rc = small ? gemm::make_problem<gemm::R4SCfg>(pbs[g], ms[g], ns[g], nseg[g], segs[g],
+                                                            gemm::kKMajor, b_layout, 0)
+                         : gemm::make_problem<gemm::R4Cfg>(pbs[g], ms[g], ns[g], nseg[g], segs[g],
+                                                           gemm::kKMajor, b_layout, 0);
+    if (rc) return rc;
+  }
   hipStream_t st = (hipStream_t)stream;
-  if (c_dtype == ML_BF16)
-    return gemm::launch_store_group<bf16>(pbs, count, b_layout, C, ldc, alpha, beta, st);
-  if (c_dtype == ML_F32)
-    return gemm::launch_store_group<float>(pbs, count, b_layout, C, ldc, alpha, beta, st);
+  auto go = [&](auto tc) {
+    using TC = decltype(tc);
+    return small ? gemm::launch_store_group<gemm::R4SCfg, TC>(pbs, count, b_layout, C, ldc, alpha,
+                                                              beta, st)
+                 : gemm::launch_store_group<gemm::R4Cfg, TC>(pbs, count, b_layout, C, ldc, alpha,
+                                                             beta, st);
+  };
+  if (c_dtype == ML_BF16) return go(bf16{});
+  if (c_dtype == ML_F32) return go(float{});
   set_error("gemm group: C dtype %d not supported (fp32 or bf16)", c_dtype);
   return ML_ERR_INVALID;
 }
@@ -164,6 +235,8 @@ extern "C" int ml_gemm_bf16_splitk(int64_t M, int64_t N, int64_t K, const void* 
     case 0: return gemm::run_splitk<gemm::BigCfg>(M, N, s, a_layout, b_layout, ksplit, C, ldc, c_dtype, alpha, beta, workspace, workspace_bytes, st);
     case 1: return gemm::run_splitk<gemm::TallCfg>(M, N, s, a_layout, b_layout, ksplit, C, ldc, c_dtype, alpha, beta, workspace, workspace_bytes, st);
     case 2: return gemm::run_splitk<gemm::WideCfg>(M, N, s, a_layout, b_layout, ksplit, C, ldc, c_dtype, alpha, beta, workspace, workspace_bytes, st);
-    default: set_error("gemm: tile_cfg must be 0 (256x256), 1 (256x32) or 2 (64x256)"); return ML_ERR_INVALID;
+    case 3: return gemm::run_splitk_r4<gemm::R4SCfg>(M, N, s, a_layout, b_layout, ksplit, C, ldc, c_dtype, alpha, beta, workspace, workspace_bytes, st);
+    case 4: return gemm::run_splitk_r4<gemm::R4Cfg>(M, N, s, a_layout, b_layout, ksplit, C, ldc, c_dtype, alpha, beta, workspace, workspace_bytes, st);
+    default: set_error("gemm: tile_cfg must be 0 (256x256), 1 (256x32), 2 (64x256), 3 (128x128) or 4 (256x256, K-major A)"); return ML_ERR_INVALID;
   }
 }

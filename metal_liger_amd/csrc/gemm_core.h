@@ -87,6 +87,7 @@ struct Cfg {
 
 using BigCfg = Cfg<256, 256, 2>;   // 2 x 4 waves of 128 x 64 (its own engine)
 using R4Cfg = Cfg<256, 256, 2, 2>; // 4 waves of 128 x 128 (the r4 engine)
+using R4SCfg = Cfg<128, 128, 2, 2>; // 4 waves of 64 x 64 (the r4 engine)
 using TallCfg = Cfg<256, 32, 4>;   // 4 x 1 waves of 64 x 32  (rank-r wide outputs)
 using WideCfg = Cfg<64, 256, 1>;   // 1 x 4 waves of 64 x 64  (few-row outputs)
 
@@ -109,8 +110,8 @@ struct Problem {
   Segment seg[kMaxSeg];
   int tiles_m, tiles_n;
   int group_m;
-  int ksplit;  // >= 1; > 1 only with one segment
-  int kps;     // k-tiles per split
+  int ksplit;  // >= 1; > 1 with several segments only on the r4 engine
+  int kps;     // k-tiles per split (counted through the segments)
 };
 
 // 16-byte chunk c of LDS row r lives at chunk c ^ swz(r).
@@ -1008,11 +1009,22 @@ constexpr int THREADS = 256;
 constexpr int BK = 64;
 constexpr int TM = 8, TN = 8;
 constexpr int WM = 128, WN = 128;
-constexpr int OP_BYTES = 256 * BK * 2;      // 32 KB: one operand of one k-tile
-constexpr int LDS_BYTES = 5 * OP_BYTES;    // five operand slots
-constexpr int LOADS = 8;                    // 1-KB loads per wave per operand per k-tile
 constexpr int EPI_BYTES = 16384;            // per wave per 128 x 64 half of its sub-tile
-static_assert(4 * 2 * EPI_BYTES <= LDS_BYTES, "epilogue LDS inside the slots");
+// A tile of T x T MFMA tiles per wave: T = 8, the 256 x 256 tile, or T = 4,
+// the 128 x 128 tile (half of each count below).
+template <int T>
+struct Geom {
+  static constexpr int W = 16 * T;                   // a wave's rows and columns
+  static constexpr int TILE = 2 * W;
+  static constexpr int OP_BYTES = TILE * BK * 2;     // one operand of one k-tile (T = 8: 32 KB)
+  static constexpr int LDS_BYTES = 5 * OP_BYTES;     // five operand slots
+  static constexpr int LOADS = T;                    // 1-KB loads per wave per operand per k-tile
+  static constexpr int KROW = 2 * TILE;              // bytes of an MN-major k-row
+  static constexpr int LANES = KROW / 16;            // lanes of a load per k-row
+  static constexpr int RPG = 64 / LANES;             // k-rows per load
+  static constexpr int WAVE_EPI = T * T * 512;       // epilogue LDS per wave
+  static_assert(4 * WAVE_EPI <= LDS_BYTES, "epilogue LDS inside the slots");
+};
 constexpr uint32_t kOob = 0x80000000u;  // past every resource range used here
 constexpr int64_t kRangeMax = 0x7FFFFFFF;
 constexpr int kRsrcFlags = 0x00020000;  // raw buffer, 32-bit data format
@@ -1040,8 +1052,9 @@ __device__ __forceinline__ uint64_t uniform_u64(uint64_t v) {
 }
 
 // Global-load state of one operand for one wave. Wave w issues, per k-tile,
-// the 1-KB groups g = w + 4 i (i < 8) of the operand tile: rows 8 g .. 8 g +
-// 7 (K-major) or k-rows 2 g, 2 g + 1 (MN-major). The uniform fields are kept
+// the 1-KB groups g = w + 4 i (i < T) of the operand tile: rows 8 g .. 8 g +
+// 7 (K-major) or the k-rows RPG g .. (MN-major: 2 of 512 B at T = 8, 4 of 256
+// B at T = 4). The uniform fields are kept
 // in SGPRs; per k-tile the cursor adds kstep to base and subtracts it from
 // range.
 template <int L>
@@ -1058,7 +1071,7 @@ struct R4Load {
 //   K-major: valid data ends with row (rows - 1 - row0), k = klen - 1; rows
 //            past it start at or after that end.
 //   MN-major: valid data ends with k-row (klen - 1 - kc), column rows - 1 - row0.
-template <int L>
+template <int L, int T>
 __device__ __forceinline__ void r4_setup(R4Load<L>& it, const Operand& op, int row0, int rows,
                                          int kc, int klen, int wave, int lane) {
   const int64_t ld = op.ld;
@@ -1079,18 +1092,21 @@ __device__ __forceinline__ void r4_setup(R4Load<L>& it, const Operand& op, int r
     it.base = uniform_u64(reinterpret_cast<uint64_t>(p + ((int64_t)kc * ld + row0) * 2));
     it.range = (int64_t)uniform_u64((uint64_t)(((int64_t)(klen - kc - 1) * ld + (rows - row0)) * 2));
     it.kstep = __builtin_amdgcn_readfirstlane((uint32_t)(r4::BK * ld * 2));
-    // group g = wave + 4 i: lane l holds k-row kr = 2 g + l / 32 = 2 wave + 8 i +
-    // l / 32, physical 16-byte slot l % 32 of it, i.e. logical 32-byte unit
-    // (slot / 2) ^ h(kr), h(kr) = (kr & 3) | ((kr >> 3) & 1) << 2 = h0 | (i & 1) << 2
-    const int kr = 2 * wave + (lane >> 5);
-    const int slot = lane & 31;
+    // group g = wave + 4 i: lane l holds k-row RPG g + l / LANES = kr + 4 RPG i,
+    // physical 16-byte slot l % LANES of it, i.e. logical 32-byte unit (slot /
+    // 2) ^ h(k-row), h(k) = (k & 3) | ((k >> 3) & 1) << 2: h depends on i's
+    // parity at T = 8 (a step of 8 k-rows) and not on i at T = 4 (16)
+    using G = r4::Geom<T>;
+    const int kr = G::RPG * wave + lane / G::LANES;
+    const int slot = lane % G::LANES;
 #pragma unroll
     for (int e = 0; e < 2; ++e) {
-      const int h = (kr & 3) | (e << 2);
+      const int ke = kr + 4 * G::RPG * e;
+      const int h = (ke & 3) | (((ke >> 3) & 1) << 2);
       const int col = 16 * ((slot >> 1) ^ h) + 8 * (slot & 1);
       it.voff[e] = col < rows - row0 ? (uint32_t)(((int64_t)kr * ld + col) * 2) : r4::kOob;
     }
-    it.istride = __builtin_amdgcn_readfirstlane((uint32_t)(8 * ld * 2));
+    it.istride = __builtin_amdgcn_readfirstlane((uint32_t)(4 * G::RPG * ld * 2));
     it.kb = 0;
   }
 }
@@ -1119,13 +1135,13 @@ __device__ __forceinline__ void r4_tile_rsrc(const R4Load<L>& it, int kc, int kl
 // Per-lane fragment read offsets of a wave sub-tile starting at row wbase.
 // K-major: one per k-step (fragment f adds 2048 f); MN-major: one per
 // fragment (the second half adds 4 k-rows, k-step 1 adds 32 k-rows).
-template <int L>
+template <int L, int T>
 struct R4Frag {
-  uint32_t a[L == kKMajor ? 2 : 8];
+  uint32_t a[L == kKMajor ? 2 : T];
 };
 
-template <int L>
-__device__ __forceinline__ void r4_frag_setup(R4Frag<L>& fa, int wbase, int lane) {
+template <int L, int T>
+__device__ __forceinline__ void r4_frag_setup(R4Frag<L, T>& fa, int wbase, int lane) {
   if constexpr (L == kKMajor) {
     const int r = lane & 15, g = lane >> 4;
 #pragma unroll
@@ -1135,23 +1151,25 @@ __device__ __forceinline__ void r4_frag_setup(R4Frag<L>& fa, int wbase, int lane
     // lane 16 G + i: k-row 8 G + i / 4, columns wbase + 16 f + 4 (i % 4) .. + 3
     const int G = lane >> 4, i = lane & 15;
     const int h = ((i >> 2) & 3) | ((G & 1) << 2);
-    const uint32_t b = (uint32_t)((8 * G + (i >> 2)) * 512 + 8 * (i & 3));
+    const uint32_t b = (uint32_t)((8 * G + (i >> 2)) * r4::Geom<T>::KROW + 8 * (i & 3));
 #pragma unroll
-    for (int f = 0; f < 8; ++f) fa.a[f] = b + (uint32_t)((((wbase >> 4) + f) ^ h) << 5);
+    for (int f = 0; f < T; ++f) fa.a[f] = b + (uint32_t)((((wbase >> 4) + f) ^ h) << 5);
   }
 }
 
 // Fragment f of k-step s (an MN-major fragment is two transposing reads,
 // combined into a fresh register).
-template <int L>
-__device__ __forceinline__ bf16x8_t r4_read_frag(const char* op, const R4Frag<L>& fa, int s, int f) {
+template <int L, int T>
+__device__ __forceinline__ bf16x8_t r4_read_frag(const char* op, const R4Frag<L, T>& fa, int s,
+                                                 int f) {
   if constexpr (L == kKMajor) {
     return *reinterpret_cast<const bf16x8_t*>(op + fa.a[s] + 2048 * f);
   } else {
     typedef __attribute__((address_space(3))) i16x4_t* lp;
-    const char* p = op + fa.a[f] + 16384 * s;
+    constexpr int KROW = r4::Geom<T>::KROW;
+    const char* p = op + fa.a[f] + 32 * KROW * s;
     const i16x4_t lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lp)(p));
-    const i16x4_t hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lp)(p + 2048));
+    const i16x4_t hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lp)(p + 4 * KROW));
     typedef short i16x8_t __attribute__((ext_vector_type(8)));
     const i16x8_t w = __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7);
     return __builtin_bit_cast(bf16x8_t, w);
@@ -1165,52 +1183,58 @@ __device__ __forceinline__ void r4_mfma(f32x4_t& acc, const bf16x8_t& a, const b
   asm volatile("v_mfma_f32_16x16x32_bf16 %0, %1, %2, %0" : "+a"(acc) : "v"(a), "v"(b));
 }
 
+template <int T>
 struct R4Frags {
-  bf16x8_t a[r4::TM], b[r4::TN];
+  bf16x8_t a[T], b[T];
 };
 
 // Main loop of the r4 engine; lds holds the five operand slots.
-// Wave w computes rows 128 (w >> 1) .. + 127 and columns 128 (w & 1) .. +
-// 127 of the block tile; acc[h][i][j] is MFMA tile (i, 4 h + j).
-template <int LA, int LB>
+// Wave w computes rows 16 T (w >> 1) .. and columns 16 T (w & 1) .. of the
+// block tile; acc[h][i][j] is MFMA tile (i, 4 h + j).
+// SPLIT: the kernel may take part of K (its epilogue writes partials);
+// otherwise the prologue holds no code for it.
+template <int LA, int LB, int T, bool SPLIT>
 __device__ __forceinline__ void r4_mainloop(const Problem& pb, int tm, int tn, int split, char* lds,
-                                            f32x4_t (&acc)[2][r4::TM][4]) {
+                                            f32x4_t (&acc)[T / 4][T][4]) {
+  using G = r4::Geom<T>;
   const int tid = threadIdx.x;
   const int lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int wm = (wave >> 1) * r4::WM;
-  const int wn = (wave & 1) * r4::WN;
-  const int m0 = tm * 256;
-  const int n0 = tn * 256;
+  const int wm = (wave >> 1) * G::W;
+  const int wn = (wave & 1) * G::W;
+  const int m0 = tm * G::TILE;
+  const int n0 = tn * G::TILE;
 #pragma unroll
-  for (int h = 0; h < 2; ++h)
+  for (int h = 0; h < T / 4; ++h)
 #pragma unroll
-    for (int i = 0; i < r4::TM; ++i)
+    for (int i = 0; i < T; ++i)
 #pragma unroll
       for (int j = 0; j < 4; ++j) acc[h][i][j] = f32x4_t{0.f, 0.f, 0.f, 0.f};
 
-  int nk, k0 = 0;
-  if (pb.ksplit > 1) {  // splits are counted in 64-wide k-tiles
-    const int total = (pb.seg[0].k_len + kBK - 1) / kBK;
-    const int first = split * pb.kps;
-    nk = total - first < pb.kps ? total - first : pb.kps;
-    k0 = first * kBK;
-  } else {
-    nk = 0;
-    for (int s = 0; s < pb.nseg; ++s) nk += (pb.seg[s].k_len + r4::BK - 1) / r4::BK;
+  int nk = 0, seg = 0, k0 = 0;
+  for (int s = 0; s < pb.nseg; ++s) nk += (pb.seg[s].k_len + r4::BK - 1) / r4::BK;
+  if (SPLIT && pb.ksplit > 1) {  // splits are ranges of the segments' 64-wide k-tiles
+    int first = split * pb.kps;
+    nk = nk - first < pb.kps ? nk - first : pb.kps;
+    for (; seg < pb.nseg - 1; ++seg) {
+      const int kt = (pb.seg[seg].k_len + r4::BK - 1) / r4::BK;
+      if (first < kt) break;
+      first -= kt;
+    }
+    k0 = first * r4::BK;
   }
   if (nk <= 0) return;  // block-uniform
 
   // Load cursor: the next k-tile to load; `loaded` k-tiles have been issued.
-  int seg = 0, kc = k0, klen = pb.seg[0].k_len, loaded = 0;
+  int kc = k0, klen = pb.seg[seg].k_len, loaded = 0;
   R4Load<LA> ia;
   R4Load<LB> ib;
-  r4_setup<LA>(ia, pb.seg[0].a, m0, pb.M, kc, klen, wave, lane);
-  r4_setup<LB>(ib, pb.seg[0].b, n0, pb.N, kc, klen, wave, lane);
-  R4Frag<LA> fa;
-  R4Frag<LB> fb;
-  r4_frag_setup<LA>(fa, wm, lane);
-  r4_frag_setup<LB>(fb, wn, lane);
+  r4_setup<LA, T>(ia, pb.seg[seg].a, m0, pb.M, kc, klen, wave, lane);
+  r4_setup<LB, T>(ib, pb.seg[seg].b, n0, pb.N, kc, klen, wave, lane);
+  R4Frag<LA, T> fa;
+  R4Frag<LB, T> fb;
+  r4_frag_setup<LA, T>(fa, wm, lane);
+  r4_frag_setup<LB, T>(fb, wn, lane);
 
   rsrc_t rsa, rsb;
   uint32_t va[2], vb[2], sa, sb;
@@ -1230,8 +1254,8 @@ __device__ __forceinline__ void r4_mainloop(const Problem& pb, int tm, int tn, i
         ++seg;
         kc = 0;
         klen = pb.seg[seg].k_len;
-        r4_setup<LA>(ia, pb.seg[seg].a, m0, pb.M, 0, klen, wave, lane);
-        r4_setup<LB>(ib, pb.seg[seg].b, n0, pb.N, 0, klen, wave, lane);
+        r4_setup<LA, T>(ia, pb.seg[seg].a, m0, pb.M, 0, klen, wave, lane);
+        r4_setup<LB, T>(ib, pb.seg[seg].b, n0, pb.N, 0, klen, wave, lane);
       } else {
         ia.base += ia.kstep;
         ia.range -= ia.kstep;
@@ -1240,7 +1264,7 @@ __device__ __forceinline__ void r4_mainloop(const Problem& pb, int tm, int tn, i
       }
     }
   };
-  // Load i (0 .. 7) of operand A (OPB false) or B of the current resources
+  // Load i (< T) of operand A (OPB false) or B of the current resources
   // into the operand slot `slot`.
   auto load = [&](auto opb, char* slot, int i) __attribute__((always_inline)) {
     char* dst = slot + (wave + 4 * i) * 1024;
@@ -1252,49 +1276,50 @@ __device__ __forceinline__ void r4_mainloop(const Problem& pb, int tm, int tn, i
   using OpA = std::integral_constant<bool, false>;
   using OpB = std::integral_constant<bool, true>;
 
-  // Five 32 KB operand slots: k-tile t in (ca, cb), t + 1 in (na, nb), and
+  // Five operand slots: k-tile t in (ca, cb), t + 1 in (na, nb), and
   // a free slot fr. Phase 0 of k-tile t loads A of t + 2 into fr; phase 1
   // (after the barrier has freed ca and cb) loads B of t + 2 into ca.
   char* ca = lds;
-  char* cb = lds + r4::OP_BYTES;
-  char* na = lds + 2 * r4::OP_BYTES;
-  char* nb = lds + 3 * r4::OP_BYTES;
-  char* fr = lds + 4 * r4::OP_BYTES;
-  R4Frags f0, f1;
+  char* cb = lds + G::OP_BYTES;
+  char* na = lds + 2 * G::OP_BYTES;
+  char* nb = lds + 3 * G::OP_BYTES;
+  char* fr = lds + 4 * G::OP_BYTES;
+  R4Frags<T> f0, f1;
   next_tile();
 #pragma unroll
-  for (int i = 0; i < r4::LOADS; ++i) load(OpA{}, ca, i);
+  for (int i = 0; i < G::LOADS; ++i) load(OpA{}, ca, i);
 #pragma unroll
-  for (int i = 0; i < r4::LOADS; ++i) load(OpB{}, cb, i);
+  for (int i = 0; i < G::LOADS; ++i) load(OpB{}, cb, i);
   next_tile();
 #pragma unroll
-  for (int i = 0; i < r4::LOADS; ++i) load(OpA{}, na, i);
+  for (int i = 0; i < G::LOADS; ++i) load(OpA{}, na, i);
 #pragma unroll
-  for (int i = 0; i < r4::LOADS; ++i) load(OpB{}, nb, i);
-  __builtin_amdgcn_s_waitcnt(big::wait_vm(2 * r4::LOADS));  // this wave's k-tile 0 landed
+  for (int i = 0; i < G::LOADS; ++i) load(OpB{}, nb, i);
+  __builtin_amdgcn_s_waitcnt(big::wait_vm(2 * G::LOADS));  // this wave's k-tile 0 landed
   lds_barrier();
 #pragma unroll
-  for (int j = 0; j < r4::TN; ++j) f0.b[j] = r4_read_frag<LB>(cb, fb, 0, j);
+  for (int j = 0; j < T; ++j) f0.b[j] = r4_read_frag<LB, T>(cb, fb, 0, j);
 #pragma unroll
-  for (int i = 0; i < r4::TM; ++i) f0.a[i] = r4_read_frag<LA>(ca, fa, 0, i);
+  for (int i = 0; i < T; ++i) f0.a[i] = r4_read_frag<LA, T>(ca, fa, 0, i);
 
-  // One phase: the 64 MFMAs of fragment set fc, with the reads of the next
+  // One phase: the T x T MFMAs of fragment set fc, with the reads of the next
   // k-step (k-step NS of slots ra_ / rb_) into fn interleaved; phase 0 moves
   // the cursor to k-tile t + 2 and issues its A loads into ld, phase 1 its
   // B loads into ld.
-  auto phase = [&](auto pc, R4Frags& fc, R4Frags& fn, const char* ra_, const char* rb_, char* ld)
+  auto phase = [&](auto pc, R4Frags<T>& fc, R4Frags<T>& fn, const char* ra_, const char* rb_, char* ld)
                    __attribute__((always_inline)) {
     constexpr int P = decltype(pc)::value;
     constexpr int NS = P ^ 1;
     if constexpr (P == 0) next_tile();
-    static_for<r4::TM * r4::TN>([&](auto qc) {
+    static_for<T * T>([&](auto qc) {
       constexpr int q = decltype(qc)::value;
-      constexpr int i = q / r4::TN, j = q % r4::TN;
-      if constexpr ((q & 1) == 0 && q < 16) fn.b[q >> 1] = r4_read_frag<LB>(rb_, fb, NS, q >> 1);
-      if constexpr ((q & 1) == 0 && q >= 16 && q < 32) fn.a[(q - 16) >> 1] = r4_read_frag<LA>(ra_, fa, NS, (q - 16) >> 1);
-      if constexpr ((q & 7) == 3) {
-        if constexpr (P == 0) load(OpA{}, ld, q >> 3);
-        else load(OpB{}, ld, q >> 3);
+      constexpr int i = q / T, j = q % T;
+      constexpr int RS = T / 4, r = q / RS;  // a read every RS slots of the first half
+      if constexpr (q % RS == 0 && r < T) fn.b[r] = r4_read_frag<LB, T>(rb_, fb, NS, r);
+      if constexpr (q % RS == 0 && r >= T && r < 2 * T) fn.a[r - T] = r4_read_frag<LA, T>(ra_, fa, NS, r - T);
+      if constexpr (q % T == 3) {
+        if constexpr (P == 0) load(OpA{}, ld, q / T);
+        else load(OpB{}, ld, q / T);
       }
       r4_mfma(acc[j >> 2][i][j & 3], fc.a[i], fc.b[j]);
       __builtin_amdgcn_sched_barrier(0);
@@ -1305,7 +1330,7 @@ __device__ __forceinline__ void r4_mainloop(const Problem& pb, int tm, int tn, i
     // this wave's loads of k-tile t + 1 have landed (only the A loads of
     // t + 2 may still be in flight); the barrier publishes them and frees
     // ca and cb
-    __builtin_amdgcn_s_waitcnt(big::wait_vm(r4::LOADS));
+    __builtin_amdgcn_s_waitcnt(big::wait_vm(G::LOADS));
     lds_barrier();
     phase(std::integral_constant<int, 1>{}, f1, f0, na, nb, ca);
     char* const oa = ca;
@@ -1539,6 +1564,8 @@ struct HasFullTile<E, std::void_t<decltype(std::declval<const E&>().full_tile(
                           std::declval<f32x4_t (&)[2][r4::TM][4]>(), 0, 0, 0,
                           static_cast<char*>(nullptr)))>> : std::true_type {};
 
+struct EpiPartial;  // the epilogue of a product split over K
+
 template <class C, int LA, int LB, class Epi>
 __global__ __launch_bounds__(C::THREADS) void gemm_kernel(const Problem pb, const Epi epi) {
   int tm, tn, split;
@@ -1548,20 +1575,22 @@ __global__ __launch_bounds__(C::THREADS) void gemm_kernel(const Problem pb, cons
   }
   const int tid = threadIdx.x;
   const int wave = tid >> 6;
-  if constexpr (C::BM == 256 && C::BN == 256 && C::ENGINE == 2) {
-    __shared__ __attribute__((aligned(16))) char lds[r4::LDS_BYTES];
-    f32x4_t acc[2][r4::TM][4];
-    r4_mainloop<LA, LB>(pb, tm, tn, split, lds, acc);
-    // each wave gets 2 x 16 KB of LDS of its own for the two 128 x 64 halves
-    // of its sub-tile
+  if constexpr (C::ENGINE == 2) {
+    constexpr int T = C::BM / 32;
+    __shared__ __attribute__((aligned(16))) char lds[r4::Geom<T>::LDS_BYTES];
+    f32x4_t acc[T / 4][T][4];
+    r4_mainloop<LA, LB, T, std::is_same_v<Epi, EpiPartial>>(pb, tm, tn, split, lds, acc);
+    // each wave gets T x T x 512 bytes of LDS of its own (T = 8: in two
+    // halves, for the two 128 x 64 halves of its sub-tile)
     const int w = __builtin_amdgcn_readfirstlane(wave);
-    char* wl = lds + w * 2 * r4::EPI_BYTES;
-    const int em = tm * 256 + (w >> 1) * r4::WM, en = tn * 256 + (w & 1) * r4::WN;
+    char* wl = lds + w * r4::Geom<T>::WAVE_EPI;
+    const int em = tm * C::BM + (w >> 1) * r4::Geom<T>::W;
+    const int en = tn * C::BN + (w & 1) * r4::Geom<T>::W;
     if constexpr (HasFullTile<Epi>::value) {
       epi.full_tile(acc, em, en, tid & 63, wl);
     } else {
       epi(acc[0], em, en, tid & 63, wl, split);
-      epi(acc[1], em, en + 64, tid & 63, wl + r4::EPI_BYTES, split);
+      if constexpr (T == 8) epi(acc[1], em, en + 64, tid & 63, wl + T * 4 * 512, split);
     }
   } else if constexpr (C::BM == 256 && C::BN == 256) {
     __shared__ __attribute__((aligned(16))) char lds[big::STAGES * big::STAGE_BYTES];
@@ -1595,8 +1624,8 @@ struct GemmGroup {
   int count;
 };
 
-template <int LA, int LB, class Epi>
-__global__ __launch_bounds__(R4Cfg::THREADS) void gemm_group_kernel(const GemmGroup<Epi> g) {
+template <class C, int LA, int LB, class Epi>
+__global__ __launch_bounds__(C::THREADS) void gemm_group_kernel(const GemmGroup<Epi> g) {
   const int bid = blockIdx.x;
   const int p = (g.count > 2 && bid >= g.first[2]) ? 2 : (g.count > 1 && bid >= g.first[1]) ? 1 : 0;
   const Problem& pb = p == 0 ? g.pb[0] : p == 1 ? g.pb[1] : g.pb[2];
@@ -1604,14 +1633,16 @@ __global__ __launch_bounds__(R4Cfg::THREADS) void gemm_group_kernel(const GemmGr
   int tm, tn, split;
   if (!tile_coords(pb, bid - g.first[p], tm, tn, split)) return;
   const int tid = threadIdx.x;
-  __shared__ __attribute__((aligned(16))) char lds[r4::LDS_BYTES];
-  f32x4_t acc[2][r4::TM][4];
-  r4_mainloop<LA, LB>(pb, tm, tn, split, lds, acc);
+  constexpr int T = C::BM / 32;
+  __shared__ __attribute__((aligned(16))) char lds[r4::Geom<T>::LDS_BYTES];
+  f32x4_t acc[T / 4][T][4];
+  r4_mainloop<LA, LB, T, false>(pb, tm, tn, split, lds, acc);
   const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
-  char* wl = lds + w * 2 * r4::EPI_BYTES;
-  const int em = tm * 256 + (w >> 1) * r4::WM, en = tn * 256 + (w & 1) * r4::WN;
+  char* wl = lds + w * r4::Geom<T>::WAVE_EPI;
+  const int em = tm * C::BM + (w >> 1) * r4::Geom<T>::W;
+  const int en = tn * C::BN + (w & 1) * r4::Geom<T>::W;
   epi(acc[0], em, en, tid & 63, wl, split);
-  epi(acc[1], em, en + 64, tid & 63, wl + r4::EPI_BYTES, split);
+  if constexpr (T == 8) epi(acc[1], em, en + 64, tid & 63, wl + T * 4 * 512, split);
 }
 
 // --------------------------------------------------------------- epilogues --
@@ -1646,6 +1677,35 @@ struct EpiStore {
                 if (m[q] < M && n[q] < N)
                   load_row8_bf16(C + (int64_t)m[q] * ldc + n[q], n[q], N, o[q]);
               }
+            }
+#pragma unroll
+            for (int q = 0; q < kStageBatch; ++q) {
+              if (m[q] >= M || n[q] >= N) continue;
+              float y[8];
+#pragma unroll
+              for (int k = 0; k < 8; ++k) y[k] = beta != 0.f ? x[q][k] + beta * o[q][k] : x[q][k];
+              store_row8_bf16(C + (int64_t)m[q] * ldc + n[q], n[q], N, y);
+            }
+          });
+    } else {
+      generic(acc, m0, n0, lane);
+    }
+  }
+
+  // 128 x 128 tile: the same, a wave's 64 x 64 sub-tile in one batch.
+  __device__ __forceinline__ void operator()(f32x4_t (&acc)[4][4], int m0, int n0, int lane,
+                                             char* lds, int) const {
+    if constexpr (std::is_same_v<TC, bf16>) {
+      stage_rows_bf16<kStageBatch, 4, 4>(
+          lds, lane, m0, n0, [&](int i, int j, int v) { return alpha * acc[i][j][v]; },
+          [&](const int (&m)[kStageBatch], const int (&n)[kStageBatch],
+              const float (&x)[kStageBatch][8]) {
+            float o[kStageBatch][8];
+            if (beta != 0.f) {
+#pragma unroll
+              for (int q = 0; q < kStageBatch; ++q)
+                if (m[q] < M && n[q] < N)
+                  load_row8_bf16(C + (int64_t)m[q] * ldc + n[q], n[q], N, o[q]);
             }
 #pragma unroll
             for (int q = 0; q < kStageBatch; ++q) {
@@ -1720,6 +1780,8 @@ __global__ __launch_bounds__(256) void reduce_partials_kernel(const float* __res
   const int64_t total = (int64_t)M * N;
   if (N % 4 == 0) {
     const int64_t nv = total / 4;
+    const bool vec = beta == 0.f && ldo % 4 == 0 &&
+                     reinterpret_cast<uintptr_t>(out) % (4 * sizeof(TC)) == 0;
     for (int64_t q = (int64_t)blockIdx.x * 256 + threadIdx.x; q < nv;
          q += (int64_t)gridDim.x * 256) {
       const int64_t e = q * 4;
@@ -1743,6 +1805,11 @@ __global__ __launch_bounds__(256) void reduce_partials_kernel(const float* __res
       const int64_t m = e / N, n = e - m * N;
       TC* p = out + m * ldo + n;
       const float a = row_scale ? alpha * row_scale[m] : alpha;
+      if (vec) {
+        const float r[4] = {a * s[0], a * s[1], a * s[2], a * s[3]};
+        store_n<TC, 4>(p, r);
+        continue;
+      }
 #pragma unroll
       for (int c = 0; c < 4; ++c) {
         float r = a * s[c];
@@ -1816,8 +1883,9 @@ inline int make_problem(Problem& pb, int M, int N, int nseg, const Segment* segs
   pb.group_m = min(group_m > 0 ? group_m : ML_GEMM_GROUP_M, pb.tiles_m);
   pb.ksplit = 1;
   pb.kps = 0;
-  if (ksplit > 1 && pb.nseg == 1) {
-    const int total = (pb.seg[0].k_len + kBK - 1) / kBK;
+  if (ksplit > 1 && (pb.nseg == 1 || (C::ENGINE == 2 && pb.nseg > 1))) {
+    int total = 0;
+    for (int s = 0; s < pb.nseg; ++s) total += (pb.seg[s].k_len + kBK - 1) / kBK;
     const int kps = (total + ksplit - 1) / ksplit;
     pb.kps = kps;
     pb.ksplit = (total + kps - 1) / kps;  // no empty splits
@@ -1851,7 +1919,7 @@ inline int launch_store(const Problem& pb, int la, int lb, void* C, int64_t ldc,
 
 // count (1..kMaxGroup) products on the r4 engine in one launch, each with the
 // store epilogue into its own C (A K-major).
-template <typename TC>
+template <class CF, typename TC>
 inline int launch_store_group(const Problem* pbs, int count, int lb, void* const* C,
                               const int64_t* ldc, float alpha, float beta, hipStream_t st) {
   ML_CHECK(count >= 1 && count <= kMaxGroup, "gemm: 1..%d grouped products (got %d)", kMaxGroup,
@@ -1867,9 +1935,9 @@ inline int launch_store_group(const Problem* pbs, int count, int lb, void* const
   }
   for (int i = count; i <= kMaxGroup; ++i) g.first[i] = blocks;
   if (lb == kKMajor)
-    gemm_group_kernel<kKMajor, kKMajor, EpiStore<TC>><<<dim3(blocks), R4Cfg::THREADS, 0, st>>>(g);
+    gemm_group_kernel<CF, kKMajor, kKMajor, EpiStore<TC>><<<dim3(blocks), CF::THREADS, 0, st>>>(g);
   else
-    gemm_group_kernel<kKMajor, kMNMajor, EpiStore<TC>><<<dim3(blocks), R4Cfg::THREADS, 0, st>>>(g);
+    gemm_group_kernel<CF, kKMajor, kMNMajor, EpiStore<TC>><<<dim3(blocks), CF::THREADS, 0, st>>>(g);
   ML_LAUNCH_CHECK();
   return ML_OK;
 }
@@ -1895,6 +1963,121 @@ inline int launch_splitk(const Problem& pb, float* ws, TC* out, int64_t ldo, flo
 
 inline size_t splitk_ws_bytes(const Problem& pb) {
   return (size_t)pb.ksplit * (size_t)pb.M * (size_t)pb.N * sizeof(float);
+}
+
+// ------------------------------------------------------ choice of the tile --
+// r4's two tiles and its split-K for a product with a K-major A. A 256 x 256
+// tile needs 256 work items to use every CU: [1777, 12320] x [12320, 2048]
+// has 56 (251 us; 92 as 4 splits of K), [200, 2064] x [2064, 2048] has 8 (50
+// us; 21 as 32 tiles of 128 x 128, 13 with K in 4). The 128 x 128 tile (80 KB
+// of LDS: two workgroups per CU) reads LDS twice as often per MFMA and is
+// 10-25% slower where there is work for every CU either way ([8192, 2064] x
+// [2064, 6144]: 270 against 205 us).
+// product_us estimates a launch of `items` work items of kt 64-wide k-tiles
+// from measurements at M = 16 .. 8192, N = 1024 .. 6144, K = 512 .. 12352 on
+// one MI355X (the choice it makes was 2% slower than the best of the
+// measured ones on average, 20% at most): whole rounds of one workgroup per
+// CU (256) or two (128), then a partly filled round, whose k-tiles run
+// faster the emptier the chip is.
+inline double product_us(int tile, int64_t items, int kt) {
+  if (tile == 256) {
+    const int64_t full = items / 256, rem = items % 256;
+    double t = full * (16.0 + 1.46 * kt);
+    if (rem) t += 10.0 + 1.25 * kt + (0.11 * kt + 4.0) * rem / 256;
+    return t;
+  }
+  const int64_t full = items / 512, rem = items % 512;
+  double t = full * (13.0 + 0.93 * kt);
+  if (rem > 256) t += 8.0 + 0.70 * kt + 0.25 * kt * (rem - 256) / 256;
+  else if (rem) t += 4.0 + 0.53 * kt + 0.05 * kt * rem / 256;
+  return t;
+}
+
+// The second launch of a split product and the traffic of its fp32 partials
+// (written once, read once, mostly within the last-level cache).
+inline double splitk_us(int splits, int64_t mn) { return 3.0 + splits * mn * 4 / 4.3e6; }
+
+struct Plan {
+  int tile, ksplit;
+};
+
+constexpr int64_t kMaxPartialBytes = 96 << 20;
+
+// Several products of one launch (count > 1) share a plan and are not split.
+inline Plan plan_products(int count, const int* M, const int* N, const int* ktiles,
+                          bool may_split) {
+  static const int kSplits[] = {1, 2, 3, 4, 6, 8, 12, 16, 24};
+  Plan best{256, 1};
+  double best_us = -1;
+  for (int tile = 256; tile >= 128; tile /= 2) {
+    int64_t tiles = 0;
+    int kt = 0;
+    for (int i = 0; i < count; ++i) {
+      tiles += (int64_t)((M[i] + tile - 1) / tile) * ((N[i] + tile - 1) / tile);
+      kt = ktiles[i] > kt ? ktiles[i] : kt;
+    }
+    for (int ks : kSplits) {
+      const int kps = (kt + ks - 1) / ks;
+      const int splits = kps > 0 ? (kt + kps - 1) / kps : 1;
+      double us = product_us(tile, tiles * splits, kps);
+      if (splits > 1) {
+        const int64_t mn = (int64_t)M[0] * N[0];
+        if (!may_split || count > 1 || kps < 2 || splits * mn * 4 > kMaxPartialBytes) break;
+        us += splitk_us(splits, mn);
+      }
+      if (best_us < 0 || us < best_us) {
+        best_us = us;
+        best = Plan{tile, splits};
+      }
+    }
+  }
+  return best;
+}
+
+inline int segment_ktiles(int nseg, const Segment* segs) {
+  int kt = 0;
+  for (int s = 0; s < nseg; ++s) kt += (segs[s].k_len + kBK - 1) / kBK;
+  return kt;
+}
+
+inline Plan plan_product(int M, int N, int nseg, const Segment* segs, bool may_split) {
+  const int kt = segment_ktiles(nseg, segs);
+  return plan_products(1, &M, &N, &kt, may_split);
+}
+
+// Partials of run_product at these sizes (0: one split).
+inline size_t product_ws_bytes(int M, int N, int ktiles) {
+  const Plan p = plan_products(1, &M, &N, &ktiles, true);
+  return p.ksplit > 1 ? (size_t)p.ksplit * M * N * sizeof(float) : 0;
+}
+
+// C = alpha * sum_s A_s B_s + beta * C with K-major A operands on the tile and
+// split the plan picks; ws null or too small: K is not split.
+template <class CF, typename TC>
+inline int run_planned(int M, int N, int nseg, const Segment* segs, int lb, int ksplit, TC* C,
+                       int64_t ldc, float alpha, float beta, float* ws, size_t ws_bytes,
+                       hipStream_t st) {
+  Problem pb;
+  int rc = make_problem<CF>(pb, M, N, nseg, segs, kKMajor, lb, 0, ksplit);
+  if (rc) return rc;
+  if (pb.ksplit == 1) return launch_store<TC, CF>(pb, kKMajor, lb, C, ldc, alpha, beta, st);
+  ML_CHECK(ws && splitk_ws_bytes(pb) <= ws_bytes, "gemm: split-K workspace too small (%zu < %zu)",
+           ws_bytes, splitk_ws_bytes(pb));
+  return lb == kKMajor
+             ? launch_splitk<CF, kKMajor, kKMajor, TC>(pb, ws, C, ldc, alpha, beta, st)
+             : launch_splitk<CF, kKMajor, kMNMajor, TC>(pb, ws, C, ldc, alpha, beta, st);
+}
+
+template <typename TC>
+inline int run_product(int M, int N, int nseg, const Segment* segs, int lb, TC* C, int64_t ldc,
+                       float alpha, float beta, float* ws, size_t ws_bytes, hipStream_t st) {
+  Plan p = plan_product(M, N, nseg, segs, ws != nullptr);
+  if (p.ksplit > 1 && (size_t)p.ksplit * M * N * sizeof(float) > ws_bytes)
+    p = plan_product(M, N, nseg, segs, false);
+  return p.tile == 128 ? run_planned<R4SCfg>(M, N, nseg, segs, lb, p.ksplit, C, ldc, alpha, beta,
+                                             ws, ws_bytes, st)
+                       : run_planned<R4Cfg>(M, N, nseg, segs, lb, p.ksplit, C, ldc, alpha, beta,
+                                            ws, ws_bytes, st);
 }
 
 }  // namespace gemm

@@ -32,6 +32,8 @@ constexpr int kTargetItems = 512;  // work items per skinny launch (~2 per CU)
 
 size_t align256(size_t b) { return (b + 255) / 256 * 256; }
 
+int ktiles(int64_t k) { return (int)((k + kBK - 1) / kBK); }
+
 int pick_ksplit(int tiles, int k_len) {
   const int ktiles = (k_len + kBK - 1) / kBK;
   int ks = (kTargetItems + tiles - 1) / (tiles > 0 ? tiles : 1);
@@ -994,6 +996,9 @@ extern "C" int ml_lora_xa(const void* X, int64_t n_tokens, int64_t in_features, 
 static size_t qkv_partial_bytes(int64_t N, int64_t in_f, const int64_t* out_f, int nadp,
                                 int64_t r) {
   size_t m = lora::skinny_ws<WideCfg>((int)(nadp * r), (int)in_f, (int)N);
+  int kt = lora::ktiles(nadp * r);  // dX: K = [out_1 | .. | nadp r]
+  for (int i = 0; i < nadp; ++i) kt += lora::ktiles(out_f[i]);
+  m = std::max(m, product_ws_bytes((int)N, (int)in_f, kt));
   if (r == lora::kDyRank) {
     int O[3];
     for (int i = 0; i < nadp; ++i) O[i] = (int)out_f[i];
@@ -1085,10 +1090,8 @@ static int adapters_bwd(const char* what, int nadp, const void* X, int64_t n_tok
     segs[i] = Segment{{static_cast<const bf16*>(dY[i]), out_features[i]},
                       {static_cast<const bf16*>(W[i]), IN}, (int)out_features[i]};
   segs[nadp] = Segment{{P, RS}, {static_cast<const bf16*>(A_stack), IN}, RS};
-  Problem pb;
-  rc = make_problem<BigCfg>(pb, N, IN, nadp + 1, segs, kKMajor, kMNMajor, 0);
-  if (rc) return rc;
-  return launch_store<bf16, R4Cfg>(pb, kKMajor, kMNMajor, dX, IN, 1.0f, 0.0f, st);
+  return run_product(N, IN, nadp + 1, segs, kMNMajor, static_cast<bf16*>(dX), IN, 1.0f, 0.0f, part,
+                     part_bytes, st);
 }
 
 extern "C" size_t ml_lora_qkv_bwd_workspace_bytes(int64_t n_tokens, int64_t in_features,
@@ -1139,6 +1142,8 @@ static size_t mlp_partial_bytes(int64_t N, int64_t H, int64_t I, int64_t r) {
   m = std::max(m, lora::skinny_ws<TallCfg>((int)N, (int)r, (int)I));   // P_G, P_U
   m = std::max(m, lora::skinny_ws<WideCfg>((int)(2 * r), (int)H, (int)N));  // dA_GU
   m = std::max(m, lora::skinny_ws<TallCfg>((int)I, (int)r, (int)N));   // dB_G, dB_U
+  m = std::max(m, product_ws_bytes((int)N, (int)I, lora::ktiles(H) + lora::ktiles(r)));  // dH
+  m = std::max(m, product_ws_bytes((int)N, (int)H, 2 * lora::ktiles(I) + lora::ktiles(2 * r)));  // dX
   if (r == lora::kDyRank) {
     const int OD[1] = {(int)H}, OGU[2] = {(int)I, (int)I};
     m = std::max(m, lora::dy_pass_ws_bytes((int)N, OD, 1));
@@ -1247,10 +1252,7 @@ extern "C" int ml_lora_mlp_bwd(const void* X, int64_t n_tokens, int64_t hidden,
   {
     Segment segs[2] = {Segment{{dy, H}, {static_cast<const bf16*>(WD), I}, H},
                        Segment{{PD, R}, {static_cast<const bf16*>(A_D), I}, R}};
-    Problem pb;
-    rc = make_problem<BigCfg>(pb, N, I, 2, segs, kKMajor, kMNMajor, 0);
-    if (rc) return rc;
-    rc = launch_store<bf16, R4Cfg>(pb, kKMajor, kMNMajor, dgate, I, 1.f, 0.f, st);
+    rc = run_product(N, I, 2, segs, kMNMajor, dgate, I, 1.f, 0.f, part, part_bytes, st);
     if (rc) return rc;
   }
   if (fused_mid) {
@@ -1301,8 +1303,6 @@ extern "C" int ml_lora_mlp_bwd(const void* X, int64_t n_tokens, int64_t hidden,
   Segment segs[3] = {Segment{{dgate, I}, {static_cast<const bf16*>(WG), H}, I},
                      Segment{{dup, I}, {static_cast<const bf16*>(WU), H}, I},
                      Segment{{PGU, R2}, {static_cast<const bf16*>(A_GU), H}, R2}};
-  Problem pb;
-  rc = make_problem<BigCfg>(pb, N, H, 3, segs, kKMajor, kMNMajor, 0);
-  if (rc) return rc;
-  return launch_store<bf16, R4Cfg>(pb, kKMajor, kMNMajor, dX, H, 1.0f, 0.0f, st);
+  return run_product(N, H, 3, segs, kMNMajor, static_cast<bf16*>(dX), H, 1.0f, 0.0f, part,
+                     part_bytes, st);
 }

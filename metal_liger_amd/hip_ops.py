@@ -7,6 +7,8 @@ These are the only callers of the HIP library; the autograd functions in
 
 from __future__ import annotations
 
+import functools
+
 import torch
 
 from . import _hip
@@ -860,6 +862,11 @@ def lora_xa(x2: torch.Tensor, a_stack: torch.Tensor) -> torch.Tensor:
                   ksplit=_ksplit_for(tiles, K))
 
 
+@functools.lru_cache(maxsize=256)
+def _segments_ws_bytes(M: int, N: int, *k_lens: int) -> int:
+    return _hip.query("ml_gemm_bf16_segments_workspace_bytes", M, N, len(k_lens), geom(k_lens))
+
+
 def lora_linear_out(x2: torch.Tensor, w: torch.Tensor, xa: torch.Tensor,
                     sb: torch.Tensor) -> torch.Tensor:
     """X W^T + XA (s B)^T as ONE K-concatenated GEMM -> [N, out] bf16."""
@@ -870,11 +877,14 @@ def lora_linear_out(x2: torch.Tensor, w: torch.Tensor, xa: torch.Tensor,
     out = torch.empty(N, out_f, dtype=torch.bfloat16, device=x2.device)
     if N == 0:
         return out
+    k_lens = geom([K, r])
+    wsb = _segments_ws_bytes(N, out_f, K, r)
+    ws = torch.empty(wsb, dtype=torch.uint8, device=x2.device) if wsb else None
     call(
-        "ml_gemm_bf16_segments", N, out_f, 2, geom([K, r]), _hip.ptrs([x2.data_ptr(), xa.data_ptr()]),
+        "ml_gemm_bf16_segments_ws", N, out_f, 2, k_lens, _hip.ptrs([x2.data_ptr(), xa.data_ptr()]),
         geom([x2.stride(0), xa.stride(0)]), _hip.ptrs([w.data_ptr(), sb.data_ptr()]),
         geom([w.stride(0), sb.stride(0)]), 0, 0, ptr(out), out.stride(0), dtype_tag(out, "out"),
-        1.0, 0.0, stream_of(x2),
+        1.0, 0.0, ptr(ws), wsb, stream_of(x2),
     )
     return out
 
