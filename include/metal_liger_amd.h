@@ -31,7 +31,7 @@
 extern "C" {
 #endif
 
-#define ML_ABI_VERSION 8
+#define ML_ABI_VERSION 9
 
 /* dtype tags */
 #define ML_F32 0
@@ -400,10 +400,26 @@ int ml_lora_mlp_bwd(const void* X, int64_t n_tokens, int64_t hidden, int64_t int
                     float* dA_D, float* dB_G, float* dB_U, float* dB_D, void* workspace,
                     size_t workspace_bytes, void* stream);
 
+/* The parameters of up to three adapters as the LoRA products read them (the
+ * casts to the activation dtype of ops/fused_lora.py:79-81 and this library's
+ * padding of ranks), `count` (1..6) matrices in one launch: matrix i is src[i]
+ * (dtype dtypes[i]), geometry[5 i ..] = rows, cols, row stride, padded rows,
+ * padded cols (a multiple of 8); dst[i] receives it dense in bf16 with zeros
+ * in the padding, scaled[i] (or null) scales[i] times that, rounded to bf16
+ * again. dst and scaled 16-byte aligned. */
+int ml_lora_pack(int count, const void* const* src, const int64_t* geometry, const int* dtypes,
+                 const float* scales, void* const* dst, void* const* scaled, void* stream);
+
+/* The way back for the adapters' gradients: `count` (1..6) fp32 matrices
+ * src[i], geometry[3 i ..] = rows, cols, row stride, each into a dense dst[i]
+ * of type `dtype`, in one launch. */
+int ml_lora_unpack(int count, const float* const* src, const int64_t* geometry, void* const* dst,
+                   int dtype, void* stream);
+
 /* X A^T for the adapters' stacked A matrices (the rank-r products of the
  * LoRA forwards: F.linear(x, A) in _lora_linear, ops/fused_lora.py:79-81):
  * X [n_tokens, in_features] bf16 (row stride ldx), A [rank_total,
- * in_features] bf16 dense, rank_total 1..64; XA [n_tokens, rank_total] bf16
+ * in_features] bf16 dense, rank_total 1..192; XA [n_tokens, rank_total] bf16
  * (row stride ldo) = X A^T with fp32 accumulation. One pass over X (no
  * split-K partials). in_features and ldx multiples of 8, X and A 16-byte
  * aligned. */

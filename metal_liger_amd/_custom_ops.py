@@ -274,6 +274,27 @@ def _(x2, w):
     return x2.new_empty((x2.shape[0], w.shape[0]), dtype=torch.bfloat16)
 
 
+@torch.library.custom_op(f"{NS}::lora_pack", mutates_args=(), device_types=_DEV)
+def lora_pack(As: List[Tensor], Bs: List[Tensor], scales: List[float], rank: int) -> Tensor:
+    return hip_ops.lora_pack(As, Bs, scales, rank)
+
+
+@lora_pack.register_fake
+def _(As, Bs, scales, rank):
+    n = rank * (sum(a.shape[1] for a in As) + 2 * sum(b.shape[0] for b in Bs))
+    return As[0].new_empty((n,), dtype=torch.bfloat16)
+
+
+@torch.library.custom_op(f"{NS}::lora_unpack", mutates_args=(), device_types=_DEV)
+def lora_unpack(flat: Tensor, spec: List[int], dtype: torch.dtype) -> Tensor:
+    return hip_ops.lora_unpack(flat, spec, dtype)
+
+
+@lora_unpack.register_fake
+def _(flat, spec, dtype):
+    return flat.new_empty((max(hip_ops.unpack_layout(spec)[1], 1),), dtype=dtype)
+
+
 @torch.library.custom_op(f"{NS}::lora_xa", mutates_args=(), device_types=_DEV)
 def lora_xa(x2: Tensor, a_stack: Tensor) -> Tensor:
     return hip_ops.lora_xa(x2, a_stack)

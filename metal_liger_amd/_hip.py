@@ -85,6 +85,14 @@ SIGNATURES: dict[str, tuple] = {
         [_i64, _i64, _i32, _i64p, ctypes.POINTER(_p), _i64p, ctypes.POINTER(_p), _i64p, _i32, _i32,
          _p, _i64, _i32, _f32, _f32, _p, _sz, _p],
     ),
+    "ml_lora_pack": (
+        _i32,
+        [_i32, ctypes.POINTER(_p), _i64p, ctypes.POINTER(_i32), ctypes.POINTER(_f32),
+         ctypes.POINTER(_p), ctypes.POINTER(_p), _p],
+    ),
+    "ml_lora_unpack": (
+        _i32, [_i32, ctypes.POINTER(_p), _i64p, ctypes.POINTER(_p), _i32, _p],
+    ),
     "ml_lora_xa": (_i32, [_p, _i64, _i64, _i64, _p, _i64, _p, _i64, _p]),
     "ml_gemm_bf16_segments_group": (
         _i32,
@@ -151,7 +159,7 @@ SIGNATURES: dict[str, tuple] = {
     ),
 }
 
-ABI_VERSION = 8
+ABI_VERSION = 9
 
 _lib = None
 _lock = threading.Lock()

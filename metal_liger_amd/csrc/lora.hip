@@ -4,10 +4,12 @@
 // reference computes (dY the output grad, X the saved input):
 //   dA = s (dY B)^T X          dB = s dY^T (X A^T)        dX += dY W + s (dY B) A
 // Here, with every product on bf16 MFMAs (fp32 accumulation):
-//   P, dB = s dY B, s dY^T XA  ONE pass over dY (dy_pass_kernel, rank 16;
-//                              XA = X A^T saved by the forward); other ranks
-//                              use two split-K skinny products
-//   dA  = P^T X                [r, in]       64x256 tiles, split-K over tokens
+//   P, dB = s dY B, s dY^T XA  ONE pass over dY (dy_pass_kernel, one job per
+//                              16 ranks; XA = X A^T saved by the forward);
+//                              ranks that are not multiples of 16 use two
+//                              split-K skinny products
+//   dA  = P^T X                [r, in]       one pass over X (ptx_pass_kernel),
+//                              else 64x256 tiles, split-K over tokens
 //   dX  = [dY_1 | .. | dY_n | P_1..n] [W_1; ..; W_n; A_1..n]
 //         ONE 256x256-tile GEMM over the K-concatenation of every adapter's
 //         dY with its W plus the stacked rank-r terms (K = sum(out) + n r).
@@ -69,11 +71,13 @@ size_t skinny_ws(int M, int N, int k_len) {
 
 // ------------------------------------------------------------- dY pass --
 // One pass over an adapter's output grad dY [N, O] (bf16) gives both rank-r
-// products that read it (rank padded to 16):
+// products that read it, for 16 of the adapter's ranks:
 //   P  = s dY B       [N, 16]    (a reduction over O)
 //   dB = s dY^T XA    [O, 16]    (a reduction over N; XA = X A^T)
-// A workgroup of 4 waves owns a 256 x 256 tile of dY (rows m0 .., columns
-// c0 ..) and streams it through LDS in chunks of 32 rows, loaded global ->
+// An adapter of rank 16 n is n jobs of one launch on the same dY (read again
+// from the last-level cache).
+// A workgroup of 4 waves owns a tile of `rows` x 256 of dY (rows m0 .., columns
+// c0 ..; dy_tile_rows) and streams it through LDS in chunks of 32 rows, loaded global ->
 // LDS three chunks ahead, each chunk laid out like the GEMM engine's
 // MN-major k-tile (32 rows of 512 B; the 32-byte unit u of row r at
 // u ^ h(r)), with the chunk's 32 XA rows (1 KB) beside it. Per chunk:
@@ -93,7 +97,7 @@ constexpr int kDyRows = 256, kDyCols = 256, kDyChunk = 32, kDyStages = 4, kDyRan
 constexpr int kDyChunkBytes = kDyChunk * kDyCols * 2;  // 16 KB
 constexpr int kDyXaBytes = kDyChunk * kDyRank * 2;     // 1 KB
 constexpr int kDyStageBytes = kDyChunkBytes + kDyXaBytes;
-constexpr int kDyMaxAdapters = 3;
+constexpr int kDyMaxJobs = 12;  // three adapters of rank 64
 // 5 loads per wave per chunk (4 x 1 KB of dY, 256 B of XA); with three
 // chunks in flight, chunk t has landed once at most 10 remain.
 constexpr int kDyWaitAhead = big::wait_vm(10);
@@ -109,29 +113,40 @@ struct DyAdapter {
 };
 
 struct DyArgs {
-  DyAdapter ad[kDyMaxAdapters];
-  int nadp, N;
+  DyAdapter ad[kDyMaxJobs];
+  int nadp, N, rows;
 };
 
 inline int dy_ctiles(int O) { return (O + kDyCols - 1) / kDyCols; }
-inline int dy_rtiles(int N) { return (N + kDyRows - 1) / kDyRows; }
+inline int dy_rtiles(int N, int rows = kDyRows) { return (N + rows - 1) / rows; }
+// Rows per tile of a launch with `ctiles` column tiles in all: 256, or fewer
+// (whole chunks) while there is not a workgroup for every CU. (Two per CU by
+// halving the rows of [8192, 2048] was slower: the dY pass 14.8 -> 16.5 us,
+// the sums of its twice as many partials 8.2 -> 10.5.)
+inline int dy_tile_rows(int N, int ctiles) {
+  int rows = kDyRows;
+  while (rows > kDyChunk && (int64_t)ctiles * dy_rtiles(N, rows) < 256) rows /= 2;
+  return rows;
+}
 inline size_t dy_ppart_bytes(int N, int O) { return (size_t)dy_ctiles(O) * N * kDyRank * 4; }
-inline size_t dy_dbpart_bytes(int N, int O) { return (size_t)dy_rtiles(N) * O * kDyRank * 4; }
+inline size_t dy_dbpart_bytes(int N, int O, int rows = kDyRows) {
+  return (size_t)dy_rtiles(N, rows) * O * kDyRank * 4;
+}
 
 __global__ __launch_bounds__(256) void dy_pass_kernel(const DyArgs args) {
   __shared__ __attribute__((aligned(16))) char lds[kDyStages * kDyStageBytes];
   __shared__ __attribute__((aligned(16))) float pred[4][kDyChunk * kDyRank];
   const int bid = blockIdx.x;
-  const int ai = (args.nadp > 2 && bid >= args.ad[2].first) ? 2
-                 : (args.nadp > 1 && bid >= args.ad[1].first) ? 1 : 0;
-  const DyAdapter& A = ai == 0 ? args.ad[0] : ai == 1 ? args.ad[1] : args.ad[2];
+  int ai = 0;
+  while (ai + 1 < args.nadp && bid >= args.ad[ai + 1].first) ++ai;
+  const DyAdapter& A = args.ad[ai];
   const int local = bid - A.first;
   const int ct = local % A.ctiles, rt = local / A.ctiles;
-  const int m0 = rt * kDyRows, c0 = ct * kDyCols;
+  const int m0 = rt * args.rows, c0 = ct * kDyCols;
   const int N = args.N, O = A.O;
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int rows = N - m0 < kDyRows ? N - m0 : kDyRows;
+  const int rows = N - m0 < args.rows ? N - m0 : args.rows;
   const int nchunks = (rows + kDyChunk - 1) / kDyChunk;
 
   // B fragments of this wave's two k-steps: lane (n = lane % 16, k group
@@ -264,7 +279,7 @@ struct DyReduceJob {
   int out_f32;
 };
 struct DyReduceArgs {
-  DyReduceJob job[2 * kDyMaxAdapters];
+  DyReduceJob job[2 * kDyMaxJobs];
 };
 
 __global__ __launch_bounds__(256) void dy_reduce_kernel(const DyReduceArgs args) {
@@ -302,8 +317,8 @@ __global__ __launch_bounds__(256) void dy_reduce_kernel(const DyReduceArgs args)
   }
 }
 
-// Host side of the dY pass for up to three adapters of one layer. ws holds
-// every adapter's partials; P_i (bf16, row stride ldp) and dB_i (fp32 [O_i,
+// Host side of the dY pass for up to kDyMaxJobs jobs of one layer. ws holds
+// every job's partials; P_i (bf16, row stride ldp) and dB_i (fp32 [O_i,
 // ldb_out]) receive s_i times the sums.
 struct DyJob {
   const bf16* dy;
@@ -320,21 +335,30 @@ struct DyJob {
   int64_t lddb;
 };
 
-inline size_t dy_pass_ws_bytes(int N, const int* O, int n) {
+// Tile rows of a dY pass over n outputs, `slices` jobs each, and its partials.
+inline int dy_pass_rows(int N, const int* O, int n, int slices) {
+  int ct = 0;
+  for (int i = 0; i < n; ++i) ct += dy_ctiles(O[i]) * slices;
+  return dy_tile_rows(N, ct);
+}
+
+inline size_t dy_pass_ws_bytes(int N, const int* O, int n, int slices = 1) {
+  const int rows = dy_pass_rows(N, O, n, slices);
   size_t b = 0;
   for (int i = 0; i < n; ++i)
-    b += align256(dy_ppart_bytes(N, O[i])) + align256(dy_dbpart_bytes(N, O[i]));
+    b += slices * (align256(dy_ppart_bytes(N, O[i])) + align256(dy_dbpart_bytes(N, O[i], rows)));
   return b;
 }
 
 inline int dy_pass(int N, const DyJob* jobs, int n, char* ws, size_t ws_bytes, hipStream_t st) {
-  ML_CHECK(n >= 1 && n <= kDyMaxAdapters, "lora dY pass: 1..3 adapters");
-  int O[kDyMaxAdapters];
+  ML_CHECK(n >= 1 && n <= kDyMaxJobs, "lora dY pass: 1..%d jobs", kDyMaxJobs);
+  int O[kDyMaxJobs];
   for (int i = 0; i < n; ++i) O[i] = jobs[i].O;
   ML_CHECK(dy_pass_ws_bytes(N, O, n) <= ws_bytes, "lora dY pass: workspace too small");
   DyArgs args{};
   args.nadp = n;
   args.N = N;
+  args.rows = dy_pass_rows(N, O, n, 1);
   int blocks = 0;
   char* w = ws;
   for (int i = 0; i < n; ++i) {
@@ -354,8 +378,8 @@ inline int dy_pass(int N, const DyJob* jobs, int n, char* ws, size_t ws_bytes, h
     a.ppart = reinterpret_cast<float*>(w);
     w += align256(dy_ppart_bytes(N, j.O));
     a.dbpart = reinterpret_cast<float*>(w);
-    w += align256(dy_dbpart_bytes(N, j.O));
-    blocks += a.ctiles * dy_rtiles(N);
+    w += align256(dy_dbpart_bytes(N, j.O, args.rows));
+    blocks += a.ctiles * dy_rtiles(N, args.rows);
   }
   dy_pass_kernel<<<dim3((unsigned)blocks), 256, 0, st>>>(args);
   ML_LAUNCH_CHECK();
@@ -364,35 +388,61 @@ inline int dy_pass(int N, const DyJob* jobs, int n, char* ws, size_t ws_bytes, h
     const DyJob& j = jobs[i];
     const DyAdapter& a = args.ad[i];
     red.job[2 * i] = DyReduceJob{a.ppart, a.ctiles, N, j.p, j.ldp, j.scale, 0};
-    red.job[2 * i + 1] = DyReduceJob{a.dbpart, dy_rtiles(N), j.O, j.db, j.lddb, j.scale, 1};
+    red.job[2 * i + 1] =
+        DyReduceJob{a.dbpart, dy_rtiles(N, args.rows), j.O, j.db, j.lddb, j.scale, 1};
   }
   dy_reduce_kernel<<<dim3(128, (unsigned)(2 * n)), 256, 0, st>>>(red);
   ML_LAUNCH_CHECK();
   return ML_OK;
 }
 
+// One adapter of rank R (a multiple of 16) as R / 16 jobs; returns their count.
+inline int dy_jobs(DyJob* jobs, const DyJob& j, int R) {
+  for (int s = 0; s < R / kDyRank; ++s) {
+    jobs[s] = j;
+    jobs[s].b += s * kDyRank;
+    jobs[s].xa += s * kDyRank;
+    jobs[s].p += s * kDyRank;
+    jobs[s].db += s * kDyRank;
+  }
+  return R / kDyRank;
+}
+
+// Ranks that run on the dY and P^T X passes (others: split-K skinny products).
+inline bool pass_rank(int64_t r) { return r % kDyRank == 0 && r <= 4 * kDyRank; }
 
 // ------------------------------------------------------------- P^T X pass --
-// dA = P^T X [RT, IN] for RT = 16, 32 or 48 stacked rank-16 adapters (X the
-// saved input or h, P the rank-r products): one pass over X. A workgroup of
-// 4 waves owns a 256 x 256 tile of X and streams it through LDS in chunks of
+// dA = P^T X [rows of P^T, IN] for stacked adapters (X the saved input or h, P
+// the rank-r products), RT = 16, 32 or 48 of the rows per workgroup
+// (blockIdx.y; X comes from the last-level cache after the first). A workgroup
+// of 4 waves owns a tile of `trows` x 256 of X and streams it through LDS in chunks of
 // 32 rows (global -> LDS, three chunks ahead; the same swizzled MN-major
 // layout as the dY pass) with the chunk's 32 rows of P beside it. Per chunk,
 // wave w: B = X columns 64 w .. 64 w + 63 (transposing reads), A = P^T (P
 // rows read from LDS), RT / 16 x 4 MFMA tiles of fp32 accumulators kept over
-// the tile's rows and written as the row tile's partial part[rtile][RT][IN];
+// the tile's rows and written into the row tile's partial part[rtile][..][IN];
 // reduce_partials_kernel sums the row tiles in a fixed order.
 constexpr int kPxRows = 256, kPxCols = 256, kPxChunk = 32, kPxStages = 4;
 
-inline int px_rtiles(int N) { return (N + kPxRows - 1) / kPxRows; }
-inline size_t ptx_pass_ws_bytes(int N, int RT, int IN) {
-  return (size_t)px_rtiles(N) * RT * IN * sizeof(float);
+inline int px_group(int RT) { return RT % 48 == 0 ? 48 : RT % 32 == 0 ? 32 : 16; }
+inline int px_ctiles(int IN) { return (IN + kPxCols - 1) / kPxCols; }
+// Rows per tile, as in the dY pass.
+inline int px_rows(int N, int RT, int IN) {
+  return dy_tile_rows(N, px_ctiles(IN) * (RT / px_group(RT)));
 }
+inline int px_rtiles(int N, int rows) { return (N + rows - 1) / rows; }
+inline size_t ptx_pass_ws_bytes(int N, int RT, int IN) {
+  return (size_t)px_rtiles(N, px_rows(N, RT, IN)) * RT * IN * sizeof(float);
+}
+static_assert(kPxRows == kDyRows && kPxChunk == kDyChunk, "the passes share dy_tile_rows");
 
 template <int RT>
 __global__ __launch_bounds__(256) void ptx_pass_kernel(const bf16* __restrict__ P, int64_t ldp,
                                                        const bf16* __restrict__ X, int64_t ldx,
-                                                       int N, int IN, float* __restrict__ part) {
+                                                       int N, int IN, int trows,
+                                                       float* __restrict__ part) {
+  P += blockIdx.y * RT;
+  const int64_t prows = (int64_t)gridDim.y * RT;  // rows of a partial
   constexpr int MT = RT / 16;
   constexpr int kXBytes = kPxChunk * kPxCols * 2;  // 16 KB
   constexpr int kPBytes = kPxChunk * RT * 2;        // 1 KB per 16 columns of P
@@ -405,10 +455,10 @@ __global__ __launch_bounds__(256) void ptx_pass_kernel(const bf16* __restrict__ 
   __shared__ __attribute__((aligned(16))) char lds[kPxStages * kStage];
   const int ctiles = (IN + kPxCols - 1) / kPxCols;
   const int ct = blockIdx.x % ctiles, rt = blockIdx.x / ctiles;
-  const int m0 = rt * kPxRows, c0 = ct * kPxCols;
+  const int m0 = rt * trows, c0 = ct * kPxCols;
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int rows = N - m0 < kPxRows ? N - m0 : kPxRows;
+  const int rows = N - m0 < trows ? N - m0 : trows;
   const int nchunks = (rows + kPxChunk - 1) / kPxChunk;
 
   // X: group g = wave + 4 i covers chunk rows 2 g, 2 g + 1 (columns clamped
@@ -495,7 +545,8 @@ __global__ __launch_bounds__(256) void ptx_pass_kernel(const bf16* __restrict__ 
       for (int v = 0; v < 4; ++v) {
         const int col = c0 + 64 * wave + 16 * f + (lane & 15);
         if (col < IN)
-          part[((int64_t)rt * RT + 16 * mt + 4 * (lane >> 4) + v) * IN + col] = acc[mt][f][v];
+          part[(rt * prows + blockIdx.y * RT + 16 * mt + 4 * (lane >> 4) + v) * IN + col] =
+              acc[mt][f][v];
       }
   __builtin_amdgcn_s_waitcnt(big::kWaitVm0);  // loads past the last chunk have landed
   __syncthreads();
@@ -504,21 +555,22 @@ __global__ __launch_bounds__(256) void ptx_pass_kernel(const bf16* __restrict__ 
 // dA [RT, IN] (fp32, row stride ldda) = P^T X.
 inline int ptx_pass(int N, const bf16* P, int64_t ldp, int RT, const bf16* X, int64_t ldx, int IN,
                     float* dA, int64_t ldda, char* ws, size_t ws_bytes, hipStream_t st) {
-  ML_CHECK(RT == 16 || RT == 32 || RT == 48, "lora P^T X pass: 16, 32 or 48 rows (got %d)", RT);
+  ML_CHECK(RT >= 16 && RT % 16 == 0, "lora P^T X pass: a multiple of 16 rows (got %d)", RT);
   ML_CHECK(IN >= 8 && IN % 8 == 0 && ldx % 8 == 0 && ldp % 8 == 0,
            "lora P^T X pass: sizes and strides must be multiples of 8");
   ML_CHECK(ptx_pass_ws_bytes(N, RT, IN) <= ws_bytes, "lora P^T X pass: workspace too small");
   float* part = reinterpret_cast<float*>(ws);
-  const unsigned blocks = (unsigned)(px_rtiles(N) * ((IN + kPxCols - 1) / kPxCols));
-  if (RT == 16)
-    ptx_pass_kernel<16><<<dim3(blocks), 256, 0, st>>>(P, ldp, X, ldx, N, IN, part);
-  else if (RT == 32)
-    ptx_pass_kernel<32><<<dim3(blocks), 256, 0, st>>>(P, ldp, X, ldx, N, IN, part);
+  const int g = px_group(RT), rows = px_rows(N, RT, IN);
+  const dim3 grid((unsigned)(px_rtiles(N, rows) * px_ctiles(IN)), (unsigned)(RT / g));
+  if (g == 16)
+    ptx_pass_kernel<16><<<grid, 256, 0, st>>>(P, ldp, X, ldx, N, IN, rows, part);
+  else if (g == 32)
+    ptx_pass_kernel<32><<<grid, 256, 0, st>>>(P, ldp, X, ldx, N, IN, rows, part);
   else
-    ptx_pass_kernel<48><<<dim3(blocks), 256, 0, st>>>(P, ldp, X, ldx, N, IN, part);
+    ptx_pass_kernel<48><<<grid, 256, 0, st>>>(P, ldp, X, ldx, N, IN, rows, part);
   ML_LAUNCH_CHECK();
-  reduce_partials_kernel<float><<<dim3(256), 256, 0, st>>>(part, px_rtiles(N), RT, IN, dA, ldda,
-                                                           1.0f, 0.f);
+  reduce_partials_kernel<float><<<dim3(256), 256, 0, st>>>(part, px_rtiles(N, rows), RT, IN, dA,
+                                                           ldda, 1.0f, 0.f);
   ML_LAUNCH_CHECK();
   return ML_OK;
 }
@@ -810,8 +862,8 @@ inline size_t mlp_mid_dapart_bytes(int N, int I) {
 }
 
 inline size_t mlp_mid_ws_bytes(int N, int I) {
-  const int O[2] = {I, I};
-  return dy_pass_ws_bytes(N, O, 2) + align256(mlp_mid_dapart_bytes(N, I));
+  return 2 * (align256(dy_ppart_bytes(N, I)) + align256(dy_dbpart_bytes(N, I))) +
+         align256(mlp_mid_dapart_bytes(N, I));
 }
 
 // Whether the fused pass takes these operands (16-byte aligned vectors).
@@ -873,83 +925,180 @@ inline int mlp_mid_pass(int N, int I, bf16* dh, bf16* dup, const bf16* gate, con
   return ML_OK;
 }
 
+// ---------------------------------------------------------- adapter pack --
+// The adapters' parameters as the products read them, in one launch: bf16,
+// ranks padded with zeros to rp,
+//   A_i [r_i, in] -> rows of a stack [.., in]    B_i [out, r_i] -> [out, rp]
+// and s_i B_i rounded once more to bf16 (the forward's operand). A thread forms
+// 8 elements of a destination row. Casting, padding, scaling and stacking as
+// separate tensor operations took 7 to 10 launches per block, each longer on
+// the host than on the GPU (24 us of GPU time and ~50 us of host time of a
+// rank-16 QKV block; one launch: 5 and 8).
+struct PackJob {
+  const void* src;   // [rows, cols], row stride ld; fp32, bf16 or fp16
+  bf16* dst;         // [drows, dcols] dense; zeros past rows / cols
+  bf16* scaled;      // scale times dst, or null
+  int64_t ld;
+  int rows, cols, drows, dcols, dtype;
+  float scale;
+};
+constexpr int kMaxPack = 6;
+struct PackArgs {
+  PackJob job[kMaxPack];
+};
+
+template <typename T>
+__device__ __forceinline__ void pack_load(const PackJob& j, int r, int c, float (&x)[8]) {
+  const T* p = static_cast<const T*>(j.src) + (int64_t)r * j.ld + c;
+  if (c + 8 <= j.cols && reinterpret_cast<uintptr_t>(p) % 16 == 0) {
+    load_n<T, 8>(p, x);
+    return;
+  }
+#pragma unroll
+  for (int k = 0; k < 8; ++k) x[k] = c + k < j.cols ? to_f32(p[k]) : 0.f;
+}
+
+__global__ __launch_bounds__(256) void pack_kernel(const PackArgs args) {
+  const PackJob& j = args.job[blockIdx.y];
+  const int per_row = j.dcols / 8;
+  const int64_t total = (int64_t)j.drows * per_row;
+  for (int64_t q = (int64_t)blockIdx.x * 256 + threadIdx.x; q < total;
+       q += (int64_t)gridDim.x * 256) {
+    const int r = (int)(q / per_row), c = (int)(q % per_row) * 8;
+    float x[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+    if (r < j.rows) {
+      if (j.dtype == ML_F32) pack_load<float>(j, r, c, x);
+      else if (j.dtype == ML_BF16) pack_load<bf16>(j, r, c, x);
+      else pack_load<f16>(j, r, c, x);
+    }
+    float y[8];
+#pragma unroll
+    for (int k = 0; k < 8; ++k) {
+      x[k] = to_f32(from_f32<bf16>(x[k]));
+      y[k] = j.scale * x[k];
+    }
+    const int64_t o = (int64_t)r * j.dcols + c;
+    store_n<bf16, 8>(j.dst + o, x);
+    if (j.scaled) store_n<bf16, 8>(j.scaled + o, y);
+  }
+}
+
+// The adapters' fp32 gradients [.., rp padded] in the adapters' own shapes and
+// dtype, in one launch: matrix i takes rows x cols of src (row stride ld) into
+// a dense dst. VEC elements of a row per thread.
+struct UnpackJob {
+  const float* src;
+  void* dst;
+  int64_t ld;
+  int rows, cols;
+};
+struct UnpackArgs {
+  UnpackJob job[kMaxPack];
+};
+
+template <typename T, int VEC>
+__global__ __launch_bounds__(256) void unpack_kernel(const UnpackArgs args) {
+  const UnpackJob& j = args.job[blockIdx.y];
+  const int per_row = j.cols / VEC;
+  const int64_t total = (int64_t)j.rows * per_row;
+  for (int64_t q = (int64_t)blockIdx.x * 256 + threadIdx.x; q < total;
+       q += (int64_t)gridDim.x * 256) {
+    const int r = (int)(q / per_row), c = (int)(q % per_row) * VEC;
+    float x[VEC];
+    load_n<float, VEC>(j.src + (int64_t)r * j.ld + c, x);
+    store_n<T, VEC>(static_cast<T*>(j.dst) + (int64_t)r * j.cols + c, x);
+  }
+}
+
 // ------------------------------------------------------------------ X A^T --
 // XA [N, R] = X [N, K] A^T for the adapters' stacked A matrices (A [R, K],
-// R <= 64): the LoRA forwards' rank-r products (F.linear(x, A) of
-// ops/fused_lora.py:79-81). A workgroup of 4 waves owns 32 rows of X; wave w
-// takes the w-th quarter of the k range in steps of 32, with the MFMA
+// R <= 192, 16 NT of its rows per blockIdx.y): the LoRA forwards' rank-r
+// products (F.linear(x, A) of ops/fused_lora.py:79-81). A workgroup of 8
+// waves owns 16 MT rows of X (MT = 2; 1 where that leaves CUs without work: a
+// wave's chain of loads is what such a launch waits for); wave w takes the w-th
+// eighth of the k range in steps of 32, with the MFMA
 // operands loaded straight from global memory in their register layout
-// (lane l: 16 bytes of row l % 16 at k offset 8 (l / 16)), and the four
+// (lane l: 16 bytes of row l % 16 at k offset 8 (l / 16)), and the
 // waves' [32, 16 NT] fp32 sums meet in LDS in a fixed order before the bf16
 // store. X is read once from HBM, A (<= 256 KB) from L2; no split-K partials
 // and no second launch. Rows past N and columns past R are not stored;
 // lanes whose k lies past K contribute zeros (K % 8 == 0).
-constexpr int kXaRows = 32;
+constexpr int kXaWaves = 8;
 
-template <int NT>
-__global__ __launch_bounds__(256) void xa_kernel(const bf16* __restrict__ X, int64_t ldx,
+template <int NT, int MT>
+__global__ __launch_bounds__(64 * kXaWaves) void xa_kernel(const bf16* __restrict__ X, int64_t ldx,
                                                  const bf16* __restrict__ A, int64_t lda, int N,
                                                  int K, int R, bf16* __restrict__ XA,
                                                  int64_t ldo) {
-  constexpr int W = kXaRows * 16 * NT;  // one wave's sums
-  __shared__ float red[4 * W];
+  constexpr int W = 16 * MT * 16 * NT;  // one wave's sums
+  __shared__ float red[kXaWaves * W];
+  A += (int64_t)blockIdx.y * 16 * NT * lda;
+  XA += blockIdx.y * 16 * NT;
+  R -= blockIdx.y * 16 * NT;
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int m0 = blockIdx.x * kXaRows;
+  const int m0 = blockIdx.x * 16 * MT;
   const int ksteps = (K + 31) / 32;
-  const int per = (ksteps + 3) / 4;
+  const int per = (ksteps + kXaWaves - 1) / kXaWaves;
   const int kb = wave * per, ke = kb + per < ksteps ? kb + per : ksteps;
   const int lr = lane & 15, lk = 8 * (lane >> 4);
   // row starts (rows past N / R re-read the last row and are not stored)
-  const bf16* x0 = X + (int64_t)(m0 + lr < N ? m0 + lr : N - 1) * ldx;
-  const bf16* x1 = X + (int64_t)(m0 + 16 + lr < N ? m0 + 16 + lr : N - 1) * ldx;
+  const bf16* xp[MT];
+#pragma unroll
+  for (int t = 0; t < MT; ++t) {
+    const int row = m0 + 16 * t + lr;
+    xp[t] = X + (int64_t)(row < N ? row : N - 1) * ldx;
+  }
   const bf16* ap[NT];
 #pragma unroll
   for (int j = 0; j < NT; ++j) ap[j] = A + (int64_t)(16 * j + lr < R ? 16 * j + lr : R - 1) * lda;
-  f32x4_t acc[2][NT];
+  f32x4_t acc[MT][NT];
 #pragma unroll
-  for (int j = 0; j < NT; ++j) acc[0][j] = acc[1][j] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+  for (int t = 0; t < MT; ++t)
+#pragma unroll
+    for (int j = 0; j < NT; ++j) acc[t][j] = f32x4_t{0.f, 0.f, 0.f, 0.f};
   const bf16x8_t zero = bf16x8_t{};
   // groups of 4 k-steps: every load of a group is in flight before its MFMAs
   // (steps past this wave's range load in-range data and are zeroed)
   for (int s0 = kb; s0 < ke; s0 += 4) {
-    bf16x8_t a0[4], a1[4], b[4][NT];
+    bf16x8_t a[4][MT], b[4][NT];
     bool ok[4];
 #pragma unroll
     for (int u = 0; u < 4; ++u) {
       const int k = 32 * (s0 + u);
       ok[u] = s0 + u < ke && k + lk < K;
       const int kc = ok[u] ? k + lk : 0;  // lanes past K read the row's first 8
-      a0[u] = *reinterpret_cast<const bf16x8_t*>(x0 + kc);
-      a1[u] = *reinterpret_cast<const bf16x8_t*>(x1 + kc);
+#pragma unroll
+      for (int t = 0; t < MT; ++t) a[u][t] = *reinterpret_cast<const bf16x8_t*>(xp[t] + kc);
 #pragma unroll
       for (int j = 0; j < NT; ++j) b[u][j] = *reinterpret_cast<const bf16x8_t*>(ap[j] + kc);
     }
 #pragma unroll
     for (int u = 0; u < 4; ++u) {
-      const bf16x8_t p0 = ok[u] ? a0[u] : zero, p1 = ok[u] ? a1[u] : zero;
 #pragma unroll
       for (int j = 0; j < NT; ++j) {
         const bf16x8_t q = ok[u] ? b[u][j] : zero;
-        acc[0][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(p0, q, acc[0][j], 0, 0, 0);
-        acc[1][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(p1, q, acc[1][j], 0, 0, 0);
+#pragma unroll
+        for (int t = 0; t < MT; ++t)
+          acc[t][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ok[u] ? a[u][t] : zero, q, acc[t][j],
+                                                              0, 0, 0);
       }
     }
   }
   // element v of tile (t, j): row 16 t + 4 (lane / 16) + v, column 16 j + lane % 16
 #pragma unroll
-  for (int t = 0; t < 2; ++t)
+  for (int t = 0; t < MT; ++t)
 #pragma unroll
     for (int j = 0; j < NT; ++j)
 #pragma unroll
       for (int v = 0; v < 4; ++v)
         red[wave * W + (16 * t + 4 * (lane >> 4) + v) * (16 * NT) + 16 * j + lr] = acc[t][j][v];
   __syncthreads();
-  for (int e = tid; e < W; e += 256) {
+  for (int e = tid; e < W; e += 64 * kXaWaves) {
     const int row = m0 + e / (16 * NT), col = e % (16 * NT);
-    if (row < N && col < R)
-      XA[(int64_t)row * ldo + col] =
-          from_f32<bf16>((red[e] + red[W + e]) + (red[2 * W + e] + red[3 * W + e]));
+    const float s = ((red[e] + red[W + e]) + (red[2 * W + e] + red[3 * W + e])) +
+                    ((red[4 * W + e] + red[5 * W + e]) + (red[6 * W + e] + red[7 * W + e]));
+    if (row < N && col < R) XA[(int64_t)row * ldo + col] = from_f32<bf16>(s);
   }
 }
 
@@ -960,6 +1109,73 @@ __global__ __launch_bounds__(256) void xa_kernel(const bf16* __restrict__ X, int
 using namespace mla;
 using namespace mla::gemm;
 
+// ---------------------------------------------------------- adapter pack --
+
+extern "C" int ml_lora_pack(int count, const void* const* src, const int64_t* geometry,
+                            const int* dtypes, const float* scales, void* const* dst,
+                            void* const* scaled, void* stream) {
+  ML_CHECK(count >= 1 && count <= lora::kMaxPack, "lora pack: 1..%d matrices (got %d)",
+           lora::kMaxPack, count);
+  ML_CHECK(src && geometry && dtypes && scales && dst && scaled, "lora pack: null argument arrays");
+  lora::PackArgs a{};
+  int64_t most = 0;
+  for (int i = 0; i < count; ++i) {
+    const int64_t* g = geometry + 5 * i;  // rows, cols, row stride, padded rows, padded cols
+    ML_CHECK(g[0] >= 0 && g[1] >= 0 && g[2] >= g[1] && g[3] >= g[0] && g[4] >= g[1] &&
+                 g[4] % 8 == 0 && g[3] < (1LL << 31) && g[4] < (1LL << 31),
+             "lora pack: bad geometry of matrix %d", i);
+    ML_CHECK(dtypes[i] == ML_F32 || dtypes[i] == ML_BF16 || dtypes[i] == ML_F16,
+             "lora pack: matrix %d must be fp32, bf16 or fp16", i);
+    ML_CHECK(dst[i] && aligned16(dst[i]) && aligned16(scaled[i]) && (src[i] || g[0] * g[1] == 0),
+             "lora pack: null or misaligned pointer for matrix %d", i);
+    a.job[i] = lora::PackJob{src[i], static_cast<bf16*>(dst[i]), static_cast<bf16*>(scaled[i]),
+                             g[2], (int)g[0], (int)g[1], (int)g[3], (int)g[4], dtypes[i],
+                             scales[i]};
+    most = std::max(most, g[3] * (g[4] / 8));
+  }
+  if (most == 0) return ML_OK;
+  const int64_t blocks = std::min<int64_t>((most + 255) / 256, 256);
+  lora::pack_kernel<<<dim3((unsigned)blocks, (unsigned)count), 256, 0, (hipStream_t)stream>>>(a);
+  ML_LAUNCH_CHECK();
+  return ML_OK;
+}
+
+extern "C" int ml_lora_unpack(int count, const float* const* src, const int64_t* geometry,
+                              void* const* dst, int dtype, void* stream) {
+  ML_CHECK(count >= 1 && count <= lora::kMaxPack, "lora unpack: 1..%d matrices (got %d)",
+           lora::kMaxPack, count);
+  ML_CHECK(src && geometry && dst, "lora unpack: null argument arrays");
+  lora::UnpackArgs a{};
+  int64_t most = 0;
+  bool vec = true;
+  for (int i = 0; i < count; ++i) {
+    const int64_t* g = geometry + 3 * i;  // rows, cols, row stride
+    ML_CHECK(g[0] >= 0 && g[1] >= 0 && g[2] >= g[1] && g[0] < (1LL << 31) && g[1] < (1LL << 31),
+             "lora unpack: bad geometry of matrix %d", i);
+    ML_CHECK((src[i] && dst[i]) || g[0] * g[1] == 0, "lora unpack: null pointer for matrix %d", i);
+    a.job[i] = lora::UnpackJob{src[i], dst[i], g[2], (int)g[0], (int)g[1]};
+    vec = vec && g[1] % 4 == 0 && g[2] % 4 == 0 && aligned16(src[i]) && aligned16(dst[i]);
+    most = std::max(most, g[0] * g[1]);
+  }
+  if (most == 0) return ML_OK;
+  const int64_t per = vec ? 1024 : 256;
+  const dim3 grid((unsigned)std::min<int64_t>((most + per - 1) / per, 512), (unsigned)count);
+  hipStream_t st = (hipStream_t)stream;
+  auto go = [&](auto t) {
+    using T = decltype(t);
+    if (vec) lora::unpack_kernel<T, 4><<<grid, 256, 0, st>>>(a);
+    else lora::unpack_kernel<T, 1><<<grid, 256, 0, st>>>(a);
+  };
+  switch (dtype) {
+    case ML_F32: go(float{}); break;
+    case ML_BF16: go(bf16{}); break;
+    case ML_F16: go(f16{}); break;
+    default: set_error("lora unpack: dtype %d not supported", dtype); return ML_ERR_INVALID;
+  }
+  ML_LAUNCH_CHECK();
+  return ML_OK;
+}
+
 // ----------------------------------------------------------------- X A^T --
 
 extern "C" int ml_lora_xa(const void* X, int64_t n_tokens, int64_t in_features, int64_t ldx,
@@ -968,7 +1184,7 @@ extern "C" int ml_lora_xa(const void* X, int64_t n_tokens, int64_t in_features, 
   ML_CHECK(n_tokens >= 0 && n_tokens < (1LL << 31), "lora xa: bad token count");
   ML_CHECK(in_features >= 8 && in_features % 8 == 0 && in_features < (1LL << 31),
            "lora xa: in_features must be a positive multiple of 8");
-  ML_CHECK(rank_total >= 1 && rank_total <= 64, "lora xa: 1..64 stacked rank rows (got %lld)",
+  ML_CHECK(rank_total >= 1 && rank_total <= 192, "lora xa: 1..192 stacked rank rows (got %lld)",
            (long long)rank_total);
   ML_CHECK(ldx >= in_features && ldx % 8 == 0 && ldo >= rank_total,
            "lora xa: bad leading dimensions");
@@ -976,17 +1192,26 @@ extern "C" int ml_lora_xa(const void* X, int64_t n_tokens, int64_t in_features, 
   ML_CHECK(X && A && XA, "lora xa: null pointer");
   ML_CHECK(aligned16(X) && aligned16(A), "lora xa: X and A must be 16-byte aligned");
   const int N = (int)n_tokens, K = (int)in_features, R = (int)rank_total;
-  const dim3 grid((unsigned)((N + lora::kXaRows - 1) / lora::kXaRows));
+  const int groups = (R + 63) / 64, nt = ((R + groups - 1) / groups + 15) / 16;
+  const unsigned gy = (unsigned)((R + 16 * nt - 1) / (16 * nt));
+  const int mt = (int64_t)((N + 31) / 32) * gy < 256 ? 1 : 2;
+  const dim3 grid((unsigned)((N + 16 * mt - 1) / (16 * mt)), gy);
   hipStream_t st = (hipStream_t)stream;
   const bf16* x = static_cast<const bf16*>(X);
   const bf16* a = static_cast<const bf16*>(A);
   bf16* o = static_cast<bf16*>(XA);
-  switch ((R + 15) / 16) {
-    case 1: lora::xa_kernel<1><<<grid, 256, 0, st>>>(x, ldx, a, K, N, K, R, o, ldo); break;
-    case 2: lora::xa_kernel<2><<<grid, 256, 0, st>>>(x, ldx, a, K, N, K, R, o, ldo); break;
-    case 3: lora::xa_kernel<3><<<grid, 256, 0, st>>>(x, ldx, a, K, N, K, R, o, ldo); break;
-    default: lora::xa_kernel<4><<<grid, 256, 0, st>>>(x, ldx, a, K, N, K, R, o, ldo); break;
+#define ML_XA(NT)                                                                                \
+  do {                                                                                           \
+    if (mt == 1) lora::xa_kernel<NT, 1><<<grid, 512, 0, st>>>(x, ldx, a, K, N, K, R, o, ldo);    \
+    else lora::xa_kernel<NT, 2><<<grid, 512, 0, st>>>(x, ldx, a, K, N, K, R, o, ldo);            \
+  } while (0)
+  switch (nt) {
+    case 1: ML_XA(1); break;
+    case 2: ML_XA(2); break;
+    case 3: ML_XA(3); break;
+    default: ML_XA(4); break;
   }
+#undef ML_XA
   ML_LAUNCH_CHECK();
   return ML_OK;
 }
@@ -999,11 +1224,11 @@ static size_t qkv_partial_bytes(int64_t N, int64_t in_f, const int64_t* out_f, i
   int kt = lora::ktiles(nadp * r);  // dX: K = [out_1 | .. | nadp r]
   for (int i = 0; i < nadp; ++i) kt += lora::ktiles(out_f[i]);
   m = std::max(m, product_ws_bytes((int)N, (int)in_f, kt));
-  if (r == lora::kDyRank) {
+  if (lora::pass_rank(r)) {
     int O[3];
     for (int i = 0; i < nadp; ++i) O[i] = (int)out_f[i];
     m = std::max(m, lora::ptx_pass_ws_bytes((int)N, (int)(nadp * r), (int)in_f));
-    return std::max(m, lora::dy_pass_ws_bytes((int)N, O, nadp));
+    return std::max(m, lora::dy_pass_ws_bytes((int)N, O, nadp, (int)r / lora::kDyRank));
   }
   for (int i = 0; i < nadp; ++i) {
     m = std::max(m, lora::skinny_ws<TallCfg>((int)N, (int)r, (int)out_f[i]));
@@ -1050,17 +1275,20 @@ static int adapters_bwd(const char* what, int nadp, const void* X, int64_t n_tok
   const bf16* x = static_cast<const bf16*>(X);
   const bf16* xa = static_cast<const bf16*>(XA);
   int rc;
-  if (R == lora::kDyRank) {
+  const bool passes = lora::pass_rank(R);
+  if (passes) {
     // P_i and dB_i of every adapter: one pass over each dY_i
-    lora::DyJob jobs[3];
+    lora::DyJob jobs[lora::kDyMaxJobs];
+    int n = 0;
     for (int i = 0; i < nadp; ++i)
-      jobs[i] = lora::DyJob{static_cast<const bf16*>(dY[i]), out_features[i],
-                            (int)out_features[i], static_cast<const bf16*>(B[i]), R, xa + i * R,
-                            RS, scale[i], P + i * R, RS, dB[i], R};
-    rc = lora::dy_pass(N, jobs, nadp, reinterpret_cast<char*>(part), part_bytes, st);
+      n += lora::dy_jobs(jobs + n,
+                         lora::DyJob{static_cast<const bf16*>(dY[i]), out_features[i],
+                                     (int)out_features[i], static_cast<const bf16*>(B[i]), R,
+                                     xa + i * R, RS, scale[i], P + i * R, RS, dB[i], R}, R);
+    rc = lora::dy_pass(N, jobs, n, reinterpret_cast<char*>(part), part_bytes, st);
     if (rc) return rc;
   }
-  for (int i = 0; i < nadp && R != lora::kDyRank; ++i) {
+  for (int i = 0; i < nadp && !passes; ++i) {
     const int OUT = (int)out_features[i];
     const bf16* dy = static_cast<const bf16*>(dY[i]);
     // P_i = s_i dY_i B_i: A = dY_i [N, out] K-major, B = B_i [out, r] (k = out, n = r) MN-major
@@ -1075,7 +1303,7 @@ static int adapters_bwd(const char* what, int nadp, const void* X, int64_t n_tok
     if (rc) return rc;
   }
   // dA_stack = P^T X: A = P^T (MN-major, ld nadp r), B = X (MN-major, ld in)
-  if (R == lora::kDyRank) {
+  if (passes) {
     rc = lora::ptx_pass(N, P, RS, RS, x, IN, IN, dA, IN, reinterpret_cast<char*>(part), part_bytes,
                         st);
   } else {
@@ -1144,10 +1372,10 @@ static size_t mlp_partial_bytes(int64_t N, int64_t H, int64_t I, int64_t r) {
   m = std::max(m, lora::skinny_ws<TallCfg>((int)I, (int)r, (int)N));   // dB_G, dB_U
   m = std::max(m, product_ws_bytes((int)N, (int)I, lora::ktiles(H) + lora::ktiles(r)));  // dH
   m = std::max(m, product_ws_bytes((int)N, (int)H, 2 * lora::ktiles(I) + lora::ktiles(2 * r)));  // dX
-  if (r == lora::kDyRank) {
-    const int OD[1] = {(int)H}, OGU[2] = {(int)I, (int)I};
-    m = std::max(m, lora::dy_pass_ws_bytes((int)N, OD, 1));
-    m = std::max(m, lora::dy_pass_ws_bytes((int)N, OGU, 2));
+  if (lora::pass_rank(r)) {
+    const int OD[1] = {(int)H}, OGU[2] = {(int)I, (int)I}, slices = (int)r / lora::kDyRank;
+    m = std::max(m, lora::dy_pass_ws_bytes((int)N, OD, 1, slices));
+    m = std::max(m, lora::dy_pass_ws_bytes((int)N, OGU, 2, slices));
     m = std::max(m, lora::ptx_pass_ws_bytes((int)N, (int)r, (int)I));
     m = std::max(m, lora::ptx_pass_ws_bytes((int)N, (int)(2 * r), (int)H));
     m = std::max(m, lora::mlp_mid_ws_bytes((int)N, (int)I));
@@ -1201,6 +1429,7 @@ extern "C" int ml_lora_mlp_bwd(const void* X, int64_t n_tokens, int64_t hidden,
   const bf16* dy = static_cast<const bf16*>(dY);
   const bf16* xa = static_cast<const bf16*>(XA_GU);
   int rc;
+  const bool passes = lora::pass_rank(R);
   // rank 16 with 16-byte aligned operands: the SwiGLU backward, the gate /
   // up adapters' P and dB, and dA_D in one pass (lora::mlp_mid_pass)
   const void* mid_ptrs[9] = {gate, up, dgate, dup, xa, PD, BG, BU, h};
@@ -1208,10 +1437,12 @@ extern "C" int ml_lora_mlp_bwd(const void* X, int64_t n_tokens, int64_t hidden,
                          lora::mlp_mid_ok(I, mid_ptrs, h ? 9 : 8, R2, R);
 
   // down projection: P_D, dA_D = P_D^T h, dB_D = s_D dY^T hA_D
-  if (R == lora::kDyRank) {  // P_D and dB_D in one pass over dY
-    const lora::DyJob jd{dy, H, H, static_cast<const bf16*>(BD), R,
-                         static_cast<const bf16*>(hA_D), R, scale[2], PD, R, dB_D, R};
-    rc = lora::dy_pass(N, &jd, 1, reinterpret_cast<char*>(part), part_bytes, st);
+  lora::DyJob jobs[lora::kDyMaxJobs];
+  if (passes) {  // P_D and dB_D in one pass over dY
+    const int n = lora::dy_jobs(jobs, lora::DyJob{dy, H, H, static_cast<const bf16*>(BD), R,
+                                                  static_cast<const bf16*>(hA_D), R, scale[2],
+                                                  PD, R, dB_D, R}, R);
+    rc = lora::dy_pass(N, jobs, n, reinterpret_cast<char*>(part), part_bytes, st);
     if (rc) return rc;
   } else {
     Segment s1{{dy, H}, {static_cast<const bf16*>(BD), R}, H};
@@ -1232,7 +1463,7 @@ extern "C" int ml_lora_mlp_bwd(const void* X, int64_t n_tokens, int64_t hidden,
   }
   if (fused_mid) {
     rc = ML_OK;  // dA_D comes from the fused pass below
-  } else if (R == lora::kDyRank) {
+  } else if (passes) {
     rc = lora::ptx_pass(N, PD, R, R, static_cast<const bf16*>(h), I, I, dA_D, I,
                         reinterpret_cast<char*>(part), part_bytes, st);
   } else {
@@ -1272,15 +1503,16 @@ extern "C" int ml_lora_mlp_bwd(const void* X, int64_t n_tokens, int64_t hidden,
   float* dBs[2] = {dB_G, dB_U};
   if (fused_mid) {
     // P_G, P_U, dB_G, dB_U came from the fused pass
-  } else if (R == lora::kDyRank) {  // P_G, P_U, dB_G, dB_U: one pass over each of d_gate, d_up
-    lora::DyJob jobs[2];
+  } else if (passes) {  // P_G, P_U, dB_G, dB_U: one pass over each of d_gate, d_up
+    int n = 0;
     for (int i = 0; i < 2; ++i)
-      jobs[i] = lora::DyJob{dgu[i], I, I, static_cast<const bf16*>(Bs[i]), R, xa + i * R, R2,
-                            scale[i], PGU + i * R, R2, dBs[i], R};
-    rc = lora::dy_pass(N, jobs, 2, reinterpret_cast<char*>(part), part_bytes, st);
+      n += lora::dy_jobs(jobs + n, lora::DyJob{dgu[i], I, I, static_cast<const bf16*>(Bs[i]), R,
+                                               xa + i * R, R2, scale[i], PGU + i * R, R2, dBs[i],
+                                               R}, R);
+    rc = lora::dy_pass(N, jobs, n, reinterpret_cast<char*>(part), part_bytes, st);
     if (rc) return rc;
   }
-  for (int i = 0; i < 2 && R != lora::kDyRank; ++i) {
+  for (int i = 0; i < 2 && !passes; ++i) {
     Segment sp{{dgu[i], I}, {static_cast<const bf16*>(Bs[i]), R}, I};
     rc = lora::skinny<TallCfg, kKMajor, kMNMajor, bf16>(N, R, sp, PGU + i * R, R2, scale[i], part,
                                                          part_bytes, st);
@@ -1290,7 +1522,7 @@ extern "C" int ml_lora_mlp_bwd(const void* X, int64_t n_tokens, int64_t hidden,
                                                            part_bytes, st);
     if (rc) return rc;
   }
-  if (R == lora::kDyRank) {
+  if (passes) {
     rc = lora::ptx_pass(N, PGU, R2, R2, x, H, H, dA_GU, H, reinterpret_cast<char*>(part),
                         part_bytes, st);
   } else {

@@ -843,13 +843,64 @@ def _ksplit_for(tiles: int, k: int) -> int:
     return max(1, min(ktiles, (512 + tiles - 1) // max(tiles, 1)))
 
 
+def lora_pack(As, Bs, scales, rank: int) -> torch.Tensor:
+    """The adapters' parameters in bf16 with ranks padded by zeros to `rank`,
+    in one buffer and one launch: every A_i [rank, in_i], then every B_i
+    [out_i, rank], then every s_i B_i. A_i [r_i, in_i], B_i [out_i, r_i] of any
+    float dtype; in_i and out_i multiples of 8."""
+    dev = ensure_rocm_device(*As, *Bs)
+    srcs, dims, tags = [], [], []
+    for i, t in enumerate((*As, *Bs)):
+        if t.dtype not in _hip.DTYPE_TAG:
+            t = t.to(torch.bfloat16)
+        if t.stride(1) != 1 or t.stride(0) < t.shape[1]:
+            t = t.contiguous()
+        r, c = t.shape
+        srcs.append(t)
+        dims += (r, c, max(t.stride(0), c), *((rank, c) if i < len(As) else (r, rank)))
+        tags.append(_hip.DTYPE_TAG[t.dtype])
+    sizes = [dims[5 * i + 3] * dims[5 * i + 4] for i in range(len(srcs))]
+    n_a, n_all = sum(sizes[:len(As)]), sum(sizes)
+    flat = torch.empty(2 * n_all - n_a, dtype=torch.bfloat16, device=dev)
+    base, dst, off = flat.data_ptr(), [], 0
+    for n in sizes:
+        dst.append(base + 2 * off)
+        off += n
+    scaled = [None] * len(As) + [p + 2 * (n_all - n_a) for p in dst[len(As):]]
+    call("ml_lora_pack", len(srcs), _hip.ptrs([t.data_ptr() for t in srcs]), geom(dims),
+         _hip.ints(tags), _hip.floats([1.0] * len(As) + list(scales)), _hip.ptrs(dst),
+         _hip.ptrs(scaled), stream_of(flat))
+    return flat
+
+
+def unpack_layout(spec):
+    """(offsets, elements) of lora_unpack's result: spec lists (source offset,
+    rows, cols, row stride) per matrix."""
+    return grad_layout([(spec[i + 1], spec[i + 2]) for i in range(0, len(spec), 4)])
+
+
+def lora_unpack(flat: torch.Tensor, spec, dtype: torch.dtype) -> torch.Tensor:
+    """Matrices of the fp32 buffer `flat` (spec: source offset, rows, cols, row
+    stride of each), dense and in `dtype`, in one buffer laid out by
+    unpack_layout and one launch."""
+    ensure_rocm_device(flat)
+    offs, total = unpack_layout(spec)
+    out = torch.empty(max(total, 1), dtype=dtype, device=flat.device)
+    src, dst, dims, es = flat.data_ptr(), out.data_ptr(), [], out.element_size()
+    for i in range(0, len(spec), 4):
+        dims += spec[i + 1:i + 4]
+    call("ml_lora_unpack", len(offs), _hip.ptrs([src + 4 * o for o in spec[::4]]), geom(dims),
+         _hip.ptrs([dst + es * o for o in offs]), _hip.DTYPE_TAG[dtype], stream_of(out))
+    return out
+
+
 def lora_xa(x2: torch.Tensor, a_stack: torch.Tensor) -> torch.Tensor:
     """X A^T for stacked LoRA A matrices: [N, in] x [R, in]^T -> [N, R] bf16.
-    Up to 64 stacked rows: one pass over X (ml_lora_xa); more: 256x32
-    tiles, split-K over in."""
+    Up to 192 stacked rows: one launch, X read once per 64 (ml_lora_xa); more:
+    256x32 tiles, split-K over in."""
     N, K = x2.shape
     R = a_stack.shape[0]
-    if R <= 64 and K % 8 == 0 and x2.stride(-1) == 1 and x2.stride(0) % 8 == 0:
+    if R <= 192 and K % 8 == 0 and x2.stride(-1) == 1 and x2.stride(0) % 8 == 0:
         out = torch.empty(N, R, dtype=torch.bfloat16, device=x2.device)
         if N == 0:
             return out

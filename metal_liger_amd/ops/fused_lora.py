@@ -4,8 +4,9 @@ X is saved once per fused block (as in the reference), and the backward of
 each block is a single call into the HIP library:
 
 * QKV (`_LoRA_QKV`): P_i = s_i dY_i B_i and dB_i = s_i dY_i^T (X A_i^T)
-  come from one streaming pass over each dY_i, dA = P^T X from one pass
-  over X (rank 16; other ranks use split-K products on narrow MFMA tiles);
+  come from one streaming pass over each dY_i per 16 ranks, dA = P^T X from
+  one pass over X per 48 stacked ranks (ranks up to 64, padded to multiples of
+  16; larger ones use split-K products on narrow MFMA tiles);
   the shared dX is ONE MFMA GEMM over the K-concatenation
   [dQ | dK | dV | P] x [Wq; Wk; Wv; A_q; A_k; A_v].
 * MLP (`_LoRA_MLP`): dH = dY W_D + s (dY B_D) A_D in one MFMA GEMM, the
@@ -34,6 +35,7 @@ import logging
 import torch
 import torch.nn as nn
 
+from metal_liger_amd import _custom_ops as _ops
 from metal_liger_amd import _custom_ops as cops
 from metal_liger_amd import hip_ops
 from metal_liger_amd._model_walk import find_layers, shadowed
@@ -100,38 +102,64 @@ def _rows_f32(t: torch.Tensor) -> torch.Tensor:
 
 
 def _pad_rank(r: int) -> int:
-    return (r + 7) // 8 * 8
+    """The rank the kernels run at: up to 64, whole 16-rank MFMA tiles (the
+    one-pass kernels over dY and X); above, multiples of 8."""
+    return (r + 15) // 16 * 16 if r <= 64 else (r + 7) // 8 * 8
 
 
-def _stack_a(As, rp: int) -> torch.Tensor:
-    """[A_1; A_2; ...] in bf16, each padded with zero rows to rp."""
-    parts = []
+def _packed(As, Bs, scales, rp: int):
+    """The adapters in bf16, ranks padded with zeros to rp: (buffer, where each
+    A_i lies in it, [B_i], [s_i B_i]). One buffer, formed in one launch; tensors that are not on a GPU (the products
+    refuse them) are formed by torch."""
+    n = len(As)
+    if As[0].is_cuda:
+        flat = _ops.lora_pack(list(As), list(Bs), scales, rp)
+    else:
+        pad = nn.functional.pad
+        a = [pad(A.detach().to(torch.bfloat16), (0, 0, 0, rp - A.shape[0])) for A in As]
+        b = [pad(B.detach().to(torch.bfloat16), (0, rp - B.shape[1])) for B in Bs]
+        flat = torch.cat([t.reshape(-1) for t in (*a, *b, *(t * s for t, s in zip(b, scales)))])
+    off, views = 0, []
     for A in As:
-        a = A.detach().to(torch.bfloat16)
-        if a.shape[0] != rp:
-            a = torch.cat([a, a.new_zeros(rp - a.shape[0], a.shape[1])], 0)
-        parts.append(a)
-    return torch.cat(parts, 0).contiguous()
+        views.append((off, rp, A.shape[1]))
+        off += rp * A.shape[1]
+    for B in (*Bs, *Bs):
+        views.append((off, B.shape[0], rp))
+        off += B.shape[0] * rp
+    mats = [_view(flat, v) for v in views[n:]]
+    return flat, views[:n], mats[:n], mats[n:]
 
 
-def _pad_b(B: torch.Tensor, rp: int, scale: float = 1.0) -> torch.Tensor:
-    """B (optionally times the LoRA scale) in bf16, padded with zero columns to rp."""
-    b = B.detach().to(torch.bfloat16)
-    if scale != 1.0:
-        b = b * scale
-    if b.shape[1] != rp:
-        b = torch.cat([b, b.new_zeros(b.shape[0], rp - b.shape[1])], 1)
-    return b.contiguous()
+def _view(flat, v):
+    off, rows, cols = v
+    return flat.as_strided((rows, cols), (cols, 1), off)
 
 
-def _adapter_grads(flat, shapes, dtypes):
-    """The adapter gradients of one fused backward call, from the fp32
-    buffer it returns (hip_ops.grad_layout): cast once to the adapters' dtype
-    when they share one, instead of autograd casting each gradient in a
-    launch of its own."""
-    if len(set(dtypes)) == 1 and dtypes[0] != flat.dtype:
+def _stack_view(flat, a_views):
+    """Consecutive A_i of one width as one [sum of rows, in] matrix."""
+    return _view(flat, (a_views[0][0], sum(v[1] for v in a_views), a_views[0][2]))
+
+
+def _adapter_grads(flat, shapes, parts, dtypes):
+    """The adapter gradients of one fused backward call, from the fp32 buffer it
+    returns (hip_ops.grad_layout of `shapes`): parts lists (which shape, first
+    row, rows, cols) of each. When the adapters share a dtype, one launch
+    brings all of them to it and to dense matrices without the ranks' padding,
+    instead of autograd casting each gradient in a launch of its own."""
+    offs, _ = hip_ops.grad_layout(shapes)
+    spec = []
+    for k, row, rows, cols in parts:
+        ld = shapes[k][1]
+        spec += (offs[k] + row * ld, rows, cols, ld)
+    groups = [spec[i:i + 4] for i in range(0, len(spec), 4)]
+    if len(set(dtypes)) == 1 and dtypes[0] in (torch.float32, torch.bfloat16, torch.float16) and (
+            dtypes[0] != flat.dtype or any(cols != ld for _, _, cols, ld in groups)):
+        if flat.is_cuda:
+            flat = _ops.lora_unpack(flat, spec, dtypes[0])
+            at, _ = hip_ops.unpack_layout(spec)
+            return [_view(flat, (o, rows, cols)) for o, (_, rows, cols, _) in zip(at, groups)]
         flat = flat.to(dtypes[0])
-    return hip_ops.grad_views(flat, shapes)
+    return [flat.as_strided((rows, cols), (ld, 1), off) for off, rows, cols, ld in groups]
 
 
 def _lora_linear(X: torch.Tensor, W: torch.Tensor,
@@ -153,9 +181,9 @@ def _lora_linear(X: torch.Tensor, W: torch.Tensor,
     if A is None or B is None:
         out = cops.linear_bf16(X2, W2)
     else:
-        rp = _pad_rank(A.shape[0])
-        xa = cops.lora_xa(X2, _stack_a([A], rp))
-        out = cops.lora_linear_out(X2, W2, xa, _pad_b(B, rp, float(scaling)))
+        flat, a_views, _, (sb,) = _packed([A], [B], [float(scaling)], _pad_rank(A.shape[0]))
+        xa = cops.lora_xa(X2, _stack_view(flat, a_views))
+        out = cops.lora_linear_out(X2, W2, xa, sb)
     return out.view(*shape[:-1], out.shape[-1])
 
 
@@ -193,12 +221,11 @@ class _LoRA_QKV(torch.autograd.Function):
         # zero gradients, which the backward slices off
         ranks = [A.shape[0] for A in (QA, KA, VA)]
         rp = _pad_rank(max(ranks))
-        a_stack = _stack_a([QA, KA, VA], rp)
+        scales = [float(QS), float(KS), float(VS)]
+        flat, a_views, Bs, sbs = _packed([QA, KA, VA], [QB, KB, VB], scales, rp)
+        a_stack = _stack_view(flat, a_views)
         xa = cops.lora_xa(Xf, a_stack)                         # [N, 3 rp], saved
         Ws = [hip_ops._bf16_rows(W.detach()) for W in (QW, KW, VW)]
-        Bs = [_pad_b(B, rp) for B in (QB, KB, VB)]
-        scales = [float(QS), float(KS), float(VS)]
-        sbs = [Bs[i] * scales[i] if scales[i] != 1.0 else Bs[i] for i in range(3)]
         # the three projections in one launch: k and v alone would each leave
         # half of the GPU idle for a round of tiles
         outs = cops.lora_qkv_out(Xf, Ws, xa, sbs)
@@ -234,12 +261,10 @@ class _LoRA_QKV(torch.autograd.Function):
         dX, flat = cops.lora_qkv_bwd(Xf, dys, [QW, KW, VW], a_stack, [QB, KB, VB],
                                      ctx.scales, xa, rp)
         shapes = hip_ops.lora_qkv_grad_shapes(Xf.shape[1], [d.shape[1] for d in dys], rp)
-        dA, *dBs = _adapter_grads(flat, shapes, [t for pair in ctx.param_dtypes for t in pair])
-        grads = []
-        for i in range(3):
-            dAi = dA[i * rp:i * rp + ranks[i]]
-            dBi = dBs[i][:, :ranks[i]]
-            grads.append((dAi, dBi))
+        parts = [(0, i * rp, r, Xf.shape[1]) for i, r in enumerate(ranks)]
+        parts += [(1 + i, 0, dys[i].shape[1], r) for i, r in enumerate(ranks)]
+        g = _adapter_grads(flat, shapes, parts, [t for pair in ctx.param_dtypes for t in pair])
+        grads = list(zip(g[:3], g[3:]))
         dX = dX.view(*shape)
         return (dX,
                 None, grads[0][0], grads[0][1], None,   # QW, QA, QB, QS
@@ -274,16 +299,16 @@ class _LoRA_MLP(torch.autograd.Function):
         ranks = [A.shape[0] for A in (GA, UA, DA)]  # padded to the largest, as in _LoRA_QKV
         rp = _pad_rank(max(ranks))
         scales = [float(GS), float(US), float(DS)]
-        a_gu = _stack_a([GA, UA], rp)                            # [2 rp, hidden]
-        a_d = _stack_a([DA], rp)                                 # [rp, inter]
+        flat, a_views, (BG, BU, BD), (sG, sU, sD) = _packed([GA, UA, DA], [GB, UB, DB], scales, rp)
+        a_gu = _stack_view(flat, a_views[:2])                    # [2 rp, hidden]
+        a_d = _stack_view(flat, a_views[2:])                     # [rp, inter]
         GWc, UWc, DWc = (hip_ops._bf16_rows(W.detach()) for W in (GW, UW, DW))
-        BG, BU, BD = (_pad_b(B, rp) for B in (GB, UB, DB))
         xa_gu = cops.lora_xa(Xf, a_gu)                            # [N, 2 rp]
-        gate = cops.lora_linear_out(Xf, GWc, xa_gu[:, :rp], BG * scales[0])
-        up = cops.lora_linear_out(Xf, UWc, xa_gu[:, rp:], BU * scales[1])
+        gate = cops.lora_linear_out(Xf, GWc, xa_gu[:, :rp], sG)
+        up = cops.lora_linear_out(Xf, UWc, xa_gu[:, rp:], sU)
         h = cops.swiglu_fwd(gate, up)                             # silu(gate) * up, bf16
         ha_d = cops.lora_xa(h, a_d)                               # [N, rp]
-        out = cops.lora_linear_out(h, DWc, ha_d, BD * scales[2])
+        out = cops.lora_linear_out(h, DWc, ha_d, sD)
         # h is not saved: the backward recomputes it from gate and up (the
         # same kernel math, so the same bits), one [N, inter] tensor less
         ctx.save_for_backward(Xf, gate, up, xa_gu, ha_d, a_gu, a_d, GWc, UWc, DWc, BG, BU, BD)
@@ -318,12 +343,15 @@ class _LoRA_MLP(torch.autograd.Function):
         dX, flat = cops.lora_mlp_bwd(
             Xf, gate, up, None, dy, GW, UW, DW, a_gu, a_d, BG, BU, BD, ctx.scales, xa_gu, ha_d, rp)
         shapes = hip_ops.lora_mlp_grad_shapes(Xf.shape[1], gate.shape[1], rp)
-        dA_GU, dA_D, dB_G, dB_U, dB_D = _adapter_grads(flat, shapes, ctx.param_dtypes)
+        H, I = Xf.shape[1], gate.shape[1]  # noqa: E741
+        parts = [(0, 0, rg, H), (0, rp, ru, H), (1, 0, rd, I), (2, 0, I, rg), (3, 0, I, ru),
+                 (4, 0, H, rd)]
+        dA_G, dA_U, dA_D, dB_G, dB_U, dB_D = _adapter_grads(flat, shapes, parts, ctx.param_dtypes)
         dX = dX.view(*shape)
         return (dX,
-                None, dA_GU[:rg], dB_G[:, :rg], None,        # GW, GA, GB, GS
-                None, dA_GU[rp:rp + ru], dB_U[:, :ru], None,  # UW, UA, UB, US
-                None, dA_D[:rd], dB_D[:, :rd], None)          # DW, DA, DB, DS
+                None, dA_G, dB_G, None,   # GW, GA, GB, GS
+                None, dA_U, dB_U, None,   # UW, UA, UB, US
+                None, dA_D, dB_D, None)   # DW, DA, DB, DS
 
 
 class _LoRA_W(torch.autograd.Function):
@@ -348,12 +376,12 @@ class _LoRA_W(torch.autograd.Function):
         Xf = hip_ops._bf16_rows(X.reshape(-1, shape[-1]))
         r = A.shape[0]
         rp = _pad_rank(r)
-        a = _stack_a([A], rp)
+        scale = float(S)
+        flat, a_views, (Bp,), (sb,) = _packed([A], [B], [scale], rp)
+        a = _stack_view(flat, a_views)
         xa = cops.lora_xa(Xf, a)                                 # [N, rp], saved
         Wc = hip_ops._bf16_rows(W.detach())
-        Bp = _pad_b(B, rp)
-        scale = float(S)
-        out = cops.lora_linear_out(Xf, Wc, xa, Bp * scale if scale != 1.0 else Bp)
+        out = cops.lora_linear_out(Xf, Wc, xa, sb)
         ctx.save_for_backward(Xf, xa, a, Wc, Bp)
         ctx.scale = scale
         ctx.param_dtypes = [A.dtype, B.dtype]
@@ -375,8 +403,9 @@ class _LoRA_W(torch.autograd.Function):
         dy = hip_ops._bf16_rows(dY.reshape(-1, dY.shape[-1]))
         dX, flat = cops.lora_linear_bwd(Xf, dy, Wc, a, Bp, ctx.scale, xa, rp)
         shapes = hip_ops.lora_linear_grad_shapes(Xf.shape[1], dy.shape[1], rp)
-        dA, dB = _adapter_grads(flat, shapes, ctx.param_dtypes)
-        return dX.view(*ctx.orig_shape), None, dA[:r], dB[:, :r], None
+        parts = [(0, 0, r, Xf.shape[1]), (1, 0, dy.shape[1], r)]
+        dA, dB = _adapter_grads(flat, shapes, parts, ctx.param_dtypes)
+        return dX.view(*ctx.orig_shape), None, dA, dB, None
 
 
 def apply_fused_lora_linear(linear, X: torch.Tensor) -> torch.Tensor:
