@@ -232,7 +232,9 @@ def floats(vals) -> ctypes.Array:
 
 
 def stream_of(t: torch.Tensor) -> int:
-    return torch.cuda.current_stream(t.device).cuda_stream
+    # the raw handle of torch.cuda.current_stream(t.device), without the Stream
+    # object (0.1 against 2.0 us per launch)
+    return torch._C._cuda_getCurrentRawStream(t.get_device())
 
 
 def dtype_tag(t: torch.Tensor, what: str) -> int:
