@@ -31,7 +31,7 @@
 extern "C" {
 #endif
 
-#define ML_ABI_VERSION 9
+#define ML_ABI_VERSION 10
 
 /* dtype tags */
 #define ML_F32 0
@@ -303,6 +303,19 @@ int ml_flce_fwd_grad(const void* hidden, int64_t ldh, const void* weight, int64_
                      int64_t vocab, int64_t hidden_size, int64_t ignore_index, int64_t token_chunk,
                      float* loss, float* lse, float* n_valid, void* d_hidden, void* d_weight,
                      void* workspace, size_t workspace_bytes, void* stream);
+
+/*
+ * The same without the tokens whose label is ignore_index, which contribute
+ * nothing: their logits are not formed, their d_hidden rows are zeros and
+ * their lse entries +inf (with which ml_flce_bwd gives zeros for them too).
+ * With both gradients NULL the same as ml_flce_fwd_grad.
+ */
+int ml_flce_fwd_grad_masked(const void* hidden, int64_t ldh, const void* weight, int64_t ldw,
+                            const void* bias, int bias_dtype, const int64_t* labels,
+                            int64_t n_tokens, int64_t vocab, int64_t hidden_size,
+                            int64_t ignore_index, int64_t token_chunk, float* loss, float* lse,
+                            float* n_valid, void* d_hidden, void* d_weight, void* workspace,
+                            size_t workspace_bytes, void* stream);
 
 /*
  * The upstream gradient of the loss (the grad_output of the reference's

@@ -196,9 +196,9 @@ def _(hidden, weight, labels, bias, ignore_index, chunk_size=8192):
 
 
 @torch.library.custom_op(f"{NS}::flce_fwd_grad", mutates_args=(), device_types=_DEV)
-def flce_fwd_grad(hidden: Tensor, weight: Tensor, labels: Tensor, bias: Optional[Tensor],
-                  ignore_index: int, need_dhidden: bool, need_dweight: bool,
-                  chunk_size: int = 8192) -> tuple[Tensor, Tensor, Tensor, Tensor, Tensor]:
+def flce_fwd_grad_all(hidden: Tensor, weight: Tensor, labels: Tensor, bias: Optional[Tensor],
+                      ignore_index: int, need_dhidden: bool, need_dweight: bool,
+                      chunk_size: int = 8192) -> tuple[Tensor, Tensor, Tensor, Tensor, Tensor]:
     loss, lse, n_valid, dh, dw = hip_ops.flce_fwd_grad(hidden, weight, labels, bias, ignore_index,
                                                        need_dhidden, need_dweight,
                                                        vocab_chunk=chunk_size)
@@ -206,6 +206,20 @@ def flce_fwd_grad(hidden: Tensor, weight: Tensor, labels: Tensor, bias: Optional
             dw if dw is not None else _none(lse))
 
 
+# What the loss Function calls: the lse of ignored tokens, which its backward
+# does not need, is not computed.
+@torch.library.custom_op(f"{NS}::flce_fwd_grad_masked", mutates_args=(), device_types=_DEV)
+def flce_fwd_grad(hidden: Tensor, weight: Tensor, labels: Tensor, bias: Optional[Tensor],
+                  ignore_index: int, need_dhidden: bool, need_dweight: bool,
+                  chunk_size: int = 8192) -> tuple[Tensor, Tensor, Tensor, Tensor, Tensor]:
+    loss, lse, n_valid, dh, dw = hip_ops.flce_fwd_grad(hidden, weight, labels, bias, ignore_index,
+                                                       need_dhidden, need_dweight,
+                                                       vocab_chunk=chunk_size, masked=True)
+    return (loss, lse, n_valid, dh if dh is not None else _none(lse),
+            dw if dw is not None else _none(lse))
+
+
+@flce_fwd_grad_all.register_fake
 @flce_fwd_grad.register_fake
 def _(hidden, weight, labels, bias, ignore_index, need_dhidden, need_dweight, chunk_size=8192):
     N, H = hidden.shape

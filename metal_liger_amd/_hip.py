@@ -116,6 +116,11 @@ SIGNATURES: dict[str, tuple] = {
         [_p, _i64, _p, _i64, _p, _i32, _p, _i64, _i64, _i64, _i64, _i64, _p, _p, _p, _p, _p, _p,
          _sz, _p],
     ),
+    "ml_flce_fwd_grad_masked": (
+        _i32,
+        [_p, _i64, _p, _i64, _p, _i32, _p, _i64, _i64, _i64, _i64, _i64, _p, _p, _p, _p, _p, _p,
+         _sz, _p],
+    ),
     "ml_flce_scale_grads": (_i32, [_p, _p, _i64, _p, _i64, _p]),
     "ml_gemm_f32_segments": (
         _i32,
@@ -159,7 +164,7 @@ SIGNATURES: dict[str, tuple] = {
     ),
 }
 
-ABI_VERSION = 9
+ABI_VERSION = 10
 
 _lib = None
 _lock = threading.Lock()

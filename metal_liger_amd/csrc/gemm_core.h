@@ -491,23 +491,24 @@ __device__ __forceinline__ void mma_tile_pipelined(f32x16_t (&acc)[C::TM][C::TN]
 // Work item of this workgroup (XCD-aware, grouped); false if none.
 // bid: the block's index among the product's blocks (blockIdx.x, or its
 // offset inside a grouped launch, whose products start at multiples of 8)
-__device__ __forceinline__ bool tile_coords(const Problem& pb, int bid, int& tm, int& tn,
-                                            int& split) {
-  const int W = pb.tiles_m * pb.tiles_n * pb.ksplit;
+__device__ __forceinline__ bool tile_coords(const Problem& pb, int tiles_m, int ksplit, int bid,
+                                            int& tm, int& tn, int& split) {
+  const int W = tiles_m * pb.tiles_n * ksplit;
   const int W8 = (W + kXcds - 1) / kXcds;
+  // (a grid may be larger than the items: the second test)
   const int logical = (bid % kXcds) * W8 + bid / kXcds;
-  if (logical >= W) return false;
+  if (logical >= W || bid / kXcds >= W8) return false;
   // the split is the slowest index: an XCD's concurrent workgroups take
   // the tiles of one K range, sharing its A rows and B columns in L2 (split
   // fastest, every tile's splits ran on one XCD and the FLCE dH product
   // re-read its 0.62 GB operands ~5x from HBM)
-  const int tiles = pb.tiles_m * pb.tiles_n;
+  const int tiles = tiles_m * pb.tiles_n;
   split = logical / tiles;
   const int t = logical - split * tiles;
   const int gsize = pb.group_m * pb.tiles_n;
   const int g = t / gsize;
   const int first_m = g * pb.group_m;
-  const int gm = min(pb.tiles_m - first_m, pb.group_m);
+  const int gm = min(tiles_m - first_m, pb.group_m);
   const int within = t - g * gsize;
   tm = first_m + within % gm;
   tn = within / gm;
@@ -850,9 +851,11 @@ __device__ __forceinline__ void big_barrier() {
 // Main loop of the big tile; lds holds STAGES stages of STAGE_BYTES (A tile,
 // then B tile). Wave w = 4 g + s computes rows 128 g .. 128 g + 127 and
 // columns 64 s .. 64 s + 63 of the block tile.
-template <int LA, int LB>
+// KLIVE: K (one segment, not split) ends at klive instead.
+template <int LA, int LB, bool KLIVE = false>
 __device__ __forceinline__ void big_mainloop(const Problem& pb, int tm, int tn, int split,
-                                             char* lds, f32x4_t (&acc)[big::TM][big::TN]) {
+                                             char* lds, f32x4_t (&acc)[big::TM][big::TN],
+                                             int klive = 0) {
   const int tid = threadIdx.x;
   const int lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -867,7 +870,9 @@ __device__ __forceinline__ void big_mainloop(const Problem& pb, int tm, int tn, 
     for (int j = 0; j < big::TN; ++j) acc[i][j] = f32x4_t{0.f, 0.f, 0.f, 0.f};
 
   int nk, k0 = 0;
-  if (pb.ksplit > 1) {  // splits are counted in 64-wide k units
+  if (KLIVE) {
+    nk = (klive + big::BK - 1) / big::BK;
+  } else if (pb.ksplit > 1) {  // splits are counted in 64-wide k units
     const int total = (pb.seg[0].k_len + kBK - 1) / kBK;
     const int first = split * pb.kps;
     const int n64 = total - first < pb.kps ? total - first : pb.kps;
@@ -884,7 +889,7 @@ __device__ __forceinline__ void big_mainloop(const Problem& pb, int tm, int tn, 
   // Load cursor: the next k-tile to load (segment seg, offset kc, length
   // klen); `loaded` k-tiles have been issued. Past the last k-tile the
   // cursor stays and every lane's load is out of range (zeros, no traffic).
-  int seg = 0, kc = k0, klen = pb.seg[0].k_len, loaded = 0;
+  int seg = 0, kc = k0, klen = KLIVE ? klive : pb.seg[0].k_len, loaded = 0;
   BigIter<LA> ia;
   BigIter<LB> ib;
   big_setup<LA>(ia, pb.seg[0].a, m0, pb.M, wave);
@@ -1194,7 +1199,8 @@ struct R4Frags {
 // SPLIT: the kernel may take part of K (its epilogue writes partials);
 // otherwise the prologue holds no code for it.
 template <int LA, int LB, int T, bool SPLIT>
-__device__ __forceinline__ void r4_mainloop(const Problem& pb, int tm, int tn, int split, char* lds,
+__device__ __forceinline__ void r4_mainloop(const Problem& pb, int tm, int tn, int split,
+                                            int ksplit, int kps, char* lds,
                                             f32x4_t (&acc)[T / 4][T][4]) {
   using G = r4::Geom<T>;
   const int tid = threadIdx.x;
@@ -1213,9 +1219,9 @@ __device__ __forceinline__ void r4_mainloop(const Problem& pb, int tm, int tn, i
 
   int nk = 0, seg = 0, k0 = 0;
   for (int s = 0; s < pb.nseg; ++s) nk += (pb.seg[s].k_len + r4::BK - 1) / r4::BK;
-  if (SPLIT && pb.ksplit > 1) {  // splits are ranges of the segments' 64-wide k-tiles
-    int first = split * pb.kps;
-    nk = nk - first < pb.kps ? nk - first : pb.kps;
+  if (SPLIT && ksplit > 1) {  // splits are ranges of the segments' 64-wide k-tiles
+    int first = split * kps;
+    nk = nk - first < kps ? nk - first : kps;
     for (; seg < pb.nseg - 1; ++seg) {
       const int kt = (pb.seg[seg].k_len + r4::BK - 1) / r4::BK;
       if (first < kt) break;
@@ -1566,10 +1572,29 @@ struct HasFullTile<E, std::void_t<decltype(std::declval<const E&>().full_tile(
 
 struct EpiPartial;  // the epilogue of a product split over K
 
+// An epilogue may fix the work on the device: live_m(pb, tiles_m, ksplit, kps)
+// lowers the number of row tiles (the rest of the grid returns at once) and may
+// split K over more workgroups instead; live_k() gives a product's K (8-wave
+// engine), 0 with nothing to store returning at once.
+template <class E, class = void>
+struct HasLiveM : std::false_type {};
+template <class E>
+struct HasLiveM<E, std::void_t<typename E::LiveM>> : std::true_type {};
+template <class E, class = void>
+struct HasLiveK : std::false_type {};
+template <class E>
+struct HasLiveK<E, std::void_t<typename E::LiveK>> : std::true_type {};
+template <class E, class = void>
+struct IsPartial : std::is_same<E, EpiPartial> {};
+template <class E>
+struct IsPartial<E, std::void_t<typename E::Partial>> : std::true_type {};
+
 template <class C, int LA, int LB, class Epi>
 __global__ __launch_bounds__(C::THREADS) void gemm_kernel(const Problem pb, const Epi epi) {
   int tm, tn, split;
-  if (!tile_coords(pb, blockIdx.x, tm, tn, split)) return;
+  int tiles_m = pb.tiles_m, ksplit = pb.ksplit, kps = pb.kps;
+  if constexpr (HasLiveM<Epi>::value) epi.live_m(pb, tiles_m, ksplit, kps);
+  if (!tile_coords(pb, tiles_m, ksplit, blockIdx.x, tm, tn, split)) return;
   if constexpr (HasSkipTile<Epi>::value) {
     if (epi.skip_tile(tm)) return;
   }
@@ -1579,7 +1604,7 @@ __global__ __launch_bounds__(C::THREADS) void gemm_kernel(const Problem pb, cons
     constexpr int T = C::BM / 32;
     __shared__ __attribute__((aligned(16))) char lds[r4::Geom<T>::LDS_BYTES];
     f32x4_t acc[T / 4][T][4];
-    r4_mainloop<LA, LB, T, std::is_same_v<Epi, EpiPartial>>(pb, tm, tn, split, lds, acc);
+    r4_mainloop<LA, LB, T, IsPartial<Epi>::value>(pb, tm, tn, split, ksplit, kps, lds, acc);
     // each wave gets T x T x 512 bytes of LDS of its own (T = 8: in two
     // halves, for the two 128 x 64 halves of its sub-tile)
     const int w = __builtin_amdgcn_readfirstlane(wave);
@@ -1595,7 +1620,13 @@ __global__ __launch_bounds__(C::THREADS) void gemm_kernel(const Problem pb, cons
   } else if constexpr (C::BM == 256 && C::BN == 256) {
     __shared__ __attribute__((aligned(16))) char lds[big::STAGES * big::STAGE_BYTES];
     f32x4_t acc[big::TM][big::TN];
-    big_mainloop<LA, LB>(pb, tm, tn, split, lds, acc);
+    if constexpr (HasLiveK<Epi>::value) {
+      const int klive = epi.live_k();
+      if (klive == 0 && epi.beta == 1.f) return;  // (block-uniform)
+      big_mainloop<LA, LB, true>(pb, tm, tn, split, lds, acc, klive);
+    } else {
+      big_mainloop<LA, LB>(pb, tm, tn, split, lds, acc);
+    }
     // each wave gets 16 KB of LDS of its own for its epilogue
     char* wl = lds + __builtin_amdgcn_readfirstlane(wave) * big::EPI_BYTES;
     epi(acc, tm * 256 + (wave >> 2) * big::WM, tn * 256 + (wave & 3) * big::WN, tid & 63, wl,
@@ -1631,12 +1662,12 @@ __global__ __launch_bounds__(C::THREADS) void gemm_group_kernel(const GemmGroup<
   const Problem& pb = p == 0 ? g.pb[0] : p == 1 ? g.pb[1] : g.pb[2];
   const Epi& epi = p == 0 ? g.epi[0] : p == 1 ? g.epi[1] : g.epi[2];
   int tm, tn, split;
-  if (!tile_coords(pb, bid - g.first[p], tm, tn, split)) return;
+  if (!tile_coords(pb, pb.tiles_m, pb.ksplit, bid - g.first[p], tm, tn, split)) return;
   const int tid = threadIdx.x;
   constexpr int T = C::BM / 32;
   __shared__ __attribute__((aligned(16))) char lds[r4::Geom<T>::LDS_BYTES];
   f32x4_t acc[T / 4][T][4];
-  r4_mainloop<LA, LB, T, false>(pb, tm, tn, split, lds, acc);
+  r4_mainloop<LA, LB, T, false>(pb, tm, tn, split, 1, 0, lds, acc);
   const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
   char* wl = lds + w * r4::Geom<T>::WAVE_EPI;
   const int em = tm * C::BM + (w >> 1) * r4::Geom<T>::W;

@@ -720,13 +720,15 @@ def flce_token_chunk(n_tokens: int, vocab: int) -> int:
 
 def flce_fwd_grad(hidden, weight, labels, bias=None, ignore_index: int = -100,
                   need_dhidden: bool = True, need_dweight: bool = True,
-                  token_chunk: int | None = None, vocab_chunk: int = 8192):
+                  token_chunk: int | None = None, vocab_chunk: int = 8192,
+                  masked: bool = False):
     """Loss and gradients for d(loss) = 1.
 
     bf16: one pass over token chunks (logits computed once); fp32: the
     reference's vocabulary-chunked schedule with vocab_chunk columns per
     chunk. Returns (loss 0-d fp32, lse [N] fp32, n_valid [1] fp32, d_hidden
-    or None, d_weight or None), gradients in the input dtype.
+    or None, d_weight or None), gradients in the input dtype. masked: bf16
+    leaves out the tokens labelled ignore_index, whose lse is +inf then.
     """
     hidden, weight, labels, bias = _flce_operands(hidden, weight, labels, bias)
     if hidden.dtype == torch.float32:
@@ -745,7 +747,7 @@ def flce_fwd_grad(hidden, weight, labels, bias=None, ignore_index: int = -100,
     wsb = _hip.query("ml_flce_fwd_grad_workspace_bytes", N, V, H, T, 1 if need_dhidden else 0)
     ws = torch.empty(max(wsb, 16), dtype=torch.uint8, device=dev)
     call(
-        "ml_flce_fwd_grad", ptr(hidden), hidden.stride(0) if N > 0 else H, ptr(weight),
+        "ml_flce_fwd_grad_masked" if masked else "ml_flce_fwd_grad", ptr(hidden), hidden.stride(0) if N > 0 else H, ptr(weight),
         weight.stride(0), ptr(bias), dtype_tag(bias, "bias") if bias is not None else 0, ptr(labels),
         N, V, H, int(ignore_index), T, ptr(loss), ptr(lse), ptr(n_valid), ptr(dh), ptr(dw), ptr(ws),
         ws.numel(), stream_of(weight),
