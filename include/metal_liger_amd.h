@@ -31,7 +31,7 @@
 extern "C" {
 #endif
 
-#define ML_ABI_VERSION 10
+#define ML_ABI_VERSION 11
 
 /* dtype tags */
 #define ML_F32 0
@@ -438,6 +438,20 @@ int ml_lora_unpack(int count, const float* const* src, const int64_t* geometry, 
  * aligned. */
 int ml_lora_xa(const void* X, int64_t n_tokens, int64_t in_features, int64_t ldx, const void* A,
                int64_t rank_total, void* XA, int64_t ldo, void* stream);
+
+/* Grouped-query attention's key / value heads (no reference counterpart: its
+ * models run transformers' attention, whose repeat_kv these replace), for
+ * `count` (1..2: k and v) tensors in one launch. geometry[10 i ..] = B, H
+ * (key / value heads), S, D, then the strides of x[i] and of y[i] over batch,
+ * head and position, in elements; D dense. Head size, strides and pointers in
+ * multiples of 16 bytes.
+ * ml_kv_expand: y[b, h groups + g, s] = x[b, h, s].
+ * ml_kv_reduce: y[b, h, s] = sum over g of x[b, h groups + g, s] (fp32 sums).
+ */
+int ml_kv_expand(int count, const void* const* x, void* const* y, const int64_t* geometry,
+                 int64_t groups, int dtype, void* stream);
+int ml_kv_reduce(int count, const void* const* x, void* const* y, const int64_t* geometry,
+                 int64_t groups, int dtype, void* stream);
 
 /* --------------------------------------------------------------------- GEMM
  * bf16 MFMA GEMM (fp32 accumulation): C = alpha * A B + beta * C.

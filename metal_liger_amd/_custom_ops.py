@@ -180,6 +180,30 @@ def _(q, k, q_weight, k_weight, cos, sin, eps, dq_out, dk_out, need_dq_weight, n
             k_weight.new_empty(k_weight.shape) if need_dk_weight else _none(dq))
 
 
+# ------------------------------------------------------ grouped-query heads --
+
+@torch.library.custom_op(f"{NS}::kv_expand", mutates_args=(), device_types=_DEV)
+def kv_expand(k: Tensor, v: Tensor, groups: int) -> tuple[Tensor, Tensor]:
+    return hip_ops.kv_expand(k, v, groups)
+
+
+@kv_expand.register_fake
+def _(k, v, groups):
+    return tuple(t.new_empty((t.shape[0], t.shape[1] * groups, t.shape[2], t.shape[3]))
+                 for t in (k, v))
+
+
+@torch.library.custom_op(f"{NS}::kv_reduce", mutates_args=(), device_types=_DEV)
+def kv_reduce(dk: Tensor, dv: Tensor, groups: int) -> tuple[Tensor, Tensor]:
+    return hip_ops.kv_reduce(dk, dv, groups)
+
+
+@kv_reduce.register_fake
+def _(dk, dv, groups):
+    return tuple(t.new_empty((t.shape[0], t.shape[2], t.shape[1] // groups,
+                              t.shape[3])).transpose(1, 2) for t in (dk, dv))
+
+
 # ------------------------------------------------------------------- FLCE --
 
 @torch.library.custom_op(f"{NS}::flce_fwd", mutates_args=(), device_types=_DEV)

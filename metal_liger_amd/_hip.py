@@ -85,6 +85,12 @@ SIGNATURES: dict[str, tuple] = {
         [_i64, _i64, _i32, _i64p, ctypes.POINTER(_p), _i64p, ctypes.POINTER(_p), _i64p, _i32, _i32,
          _p, _i64, _i32, _f32, _f32, _p, _sz, _p],
     ),
+    "ml_kv_expand": (
+        _i32, [_i32, ctypes.POINTER(_p), ctypes.POINTER(_p), _i64p, _i64, _i32, _p],
+    ),
+    "ml_kv_reduce": (
+        _i32, [_i32, ctypes.POINTER(_p), ctypes.POINTER(_p), _i64p, _i64, _i32, _p],
+    ),
     "ml_lora_pack": (
         _i32,
         [_i32, ctypes.POINTER(_p), _i64p, ctypes.POINTER(_i32), ctypes.POINTER(_f32),
@@ -164,7 +170,7 @@ SIGNATURES: dict[str, tuple] = {
     ),
 }
 
-ABI_VERSION = 10
+ABI_VERSION = 11
 
 _lib = None
 _lock = threading.Lock()

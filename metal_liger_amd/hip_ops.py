@@ -477,6 +477,50 @@ def qk_norm_rope_bwd(q: torch.Tensor, k: torch.Tensor, q_weight: torch.Tensor,
     return dq, dk, dwq, dwk
 
 
+# ------------------------------------------------------ grouped-query heads --
+
+
+def _kv_rows(t: torch.Tensor) -> torch.Tensor:
+    """[B, H, S, D] with dense rows and strides and base in multiples of 16 bytes."""
+    v = 16 // t.element_size()
+    if t.stride(3) != 1 or any(s % v for s in t.stride()[:3]) or t.data_ptr() % 16:
+        t = t.clone(memory_format=torch.contiguous_format)
+    return t
+
+
+def _kv_call(name: str, xs, ys, heads: int, groups: int):
+    dims = []
+    for x, y in zip(xs, ys):
+        dims += (x.shape[0], heads, x.shape[2], x.shape[3], *x.stride()[:3], *y.stride()[:3])
+    call(name, len(xs), _hip.ptrs([t.data_ptr() for t in xs]),
+         _hip.ptrs([t.data_ptr() for t in ys]), geom(dims), groups, dtype_tag(xs[0], "key"),
+         stream_of(xs[0]))
+
+
+def kv_expand(k: torch.Tensor, v: torch.Tensor, groups: int):
+    """k, v [B, Hkv, S, D] with every head repeated `groups` times: contiguous
+    [B, Hkv * groups, S, D] (transformers' repeat_kv), in one launch. D a
+    multiple of 16 bytes; k and v of one dtype."""
+    ensure_rocm_device(k, v)
+    xs = [_kv_rows(k), _kv_rows(v)]
+    ys = [torch.empty(t.shape[0], t.shape[1] * groups, t.shape[2], t.shape[3], dtype=t.dtype,
+                      device=t.device) for t in xs]
+    _kv_call("ml_kv_expand", xs, ys, k.shape[1], groups)
+    return tuple(ys)
+
+
+def kv_reduce(dk: torch.Tensor, dv: torch.Tensor, groups: int):
+    """The gradients of kv_expand's inputs: sums over each head's `groups`
+    copies (in fp32), as [B, Hkv, S, D] views of [B, S, Hkv, D] memory."""
+    ensure_rocm_device(dk, dv)
+    xs = [_kv_rows(dk), _kv_rows(dv)]
+    heads = dk.shape[1] // groups
+    ys = [torch.empty(t.shape[0], t.shape[2], heads, t.shape[3], dtype=t.dtype,
+                      device=t.device).transpose(1, 2) for t in xs]
+    _kv_call("ml_kv_reduce", xs, ys, heads, groups)
+    return tuple(ys)
+
+
 # -------------------------------------------------------------------- GEMM --
 
 

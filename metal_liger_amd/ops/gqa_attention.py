@@ -21,7 +21,10 @@ allowed.
 """
 
 import torch
+from torch.autograd import forward_ad
 from torch.nn.attention import SDPBackend, sdpa_kernel
+
+from metal_liger_amd import _custom_ops as cops
 
 ATTN_KEY = "metal_liger_sdpa"
 
@@ -35,6 +38,40 @@ def _repeat_heads(x: torch.Tensor, groups: int) -> torch.Tensor:
     key / value head h // groups)."""
     b, h, s, d = x.shape
     return x[:, :, None].expand(b, h, groups, s, d).reshape(b, h * groups, s, d)
+
+
+class _RepeatKV(torch.autograd.Function):
+    """_repeat_heads of key and value in one launch, and of their gradients'
+    sums in another."""
+
+    @staticmethod
+    def forward(ctx, key, value, groups):
+        ctx.groups = groups
+        return cops.kv_expand(key, value, groups)
+
+    @staticmethod
+    def backward(ctx, dk, dv):
+        dk, dv = cops.kv_reduce(dk, dv, ctx.groups)
+        return dk, dv, None
+
+
+def _repeat_kv(key: torch.Tensor, value: torch.Tensor, groups: int):
+    """key and value with their heads repeated: by the kernels for plain GPU
+    tensors in eager mode, else (other devices and dtypes, ragged head sizes,
+    torch.compile, functorch transforms, forward-mode AD) by _repeat_heads,
+    which every transform can see through."""
+    row = 16 // key.element_size()
+    if (key.is_cuda and value.is_cuda and key.dtype == value.dtype
+            and key.dtype in (torch.bfloat16, torch.float16, torch.float32)
+            and type(key) is torch.Tensor and type(value) is torch.Tensor
+            and key.dim() == 4 and key.shape[:3] == value.shape[:3]
+            and key.shape[3] % row == 0 and value.shape[3] % row == 0
+            and key.numel() > 0 and value.numel() > 0
+            and not torch.compiler.is_compiling()
+            and not torch._C._are_functorch_transforms_active()
+            and forward_ad._current_level < 0):
+        return _RepeatKV.apply(key, value, groups)
+    return _repeat_heads(key, groups), _repeat_heads(value, groups)
 
 
 def expanded_kv_attention_forward(module, query, key, value, attention_mask, dropout=0.0,
@@ -53,8 +90,7 @@ def expanded_kv_attention_forward(module, query, key, value, attention_mask, dro
                                       scaling=scaling, is_causal=is_causal, **kwargs)
     groups = getattr(module, "num_key_value_groups", 1)
     if groups > 1:
-        key = _repeat_heads(key, groups)
-        value = _repeat_heads(value, groups)
+        key, value = _repeat_kv(key, value, groups)
     q_len, kv_len = query.shape[2], key.shape[2]
     if attention_mask is not None and attention_mask.ndim == 4:
         attention_mask = attention_mask[:, :, :, :kv_len]  # as transformers' sdpa path
