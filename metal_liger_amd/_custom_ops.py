@@ -363,6 +363,37 @@ def _(x2, ws, xa, sbs):
     return [x2.new_empty((x2.shape[0], w.shape[0]), dtype=torch.bfloat16) for w in ws]
 
 
+@torch.library.custom_op(f"{NS}::lora_qkv_fwd", mutates_args=(), device_types=_DEV)
+def lora_qkv_fwd(x2: Tensor, ws: List[Tensor], As: List[Tensor], Bs: List[Tensor],
+                 scales: List[float],
+                 rank: int) -> tuple[Tensor, Tensor, Tensor, Tensor, Tensor]:
+    outs, xa, packed = hip_ops.lora_qkv_fwd(x2, ws, As, Bs, scales, rank)
+    return (*outs, xa, packed)
+
+
+@lora_qkv_fwd.register_fake
+def _(x2, ws, As, Bs, scales, rank):
+    new = lambda *s: x2.new_empty(s, dtype=torch.bfloat16)  # noqa: E731
+    n = rank * (sum(a.shape[1] for a in As) + 2 * sum(b.shape[0] for b in Bs))
+    return (*(new(x2.shape[0], w.shape[0]) for w in ws), new(x2.shape[0], 3 * rank), new(n))
+
+
+@torch.library.custom_op(f"{NS}::lora_qkv_bwd_packed", mutates_args=(), device_types=_DEV)
+def lora_qkv_bwd_packed(x2: Tensor, dys: List[Tensor], ws: List[Tensor], packed: Tensor,
+                        scales: List[float], xa: Tensor, rank: int, spec: List[int],
+                        dtype: torch.dtype) -> tuple[Tensor, Tensor]:
+    return hip_ops.lora_qkv_bwd_packed(x2, dys, ws, packed, scales, xa, rank, spec, dtype)
+
+
+@lora_qkv_bwd_packed.register_fake
+def _(x2, dys, ws, packed, scales, xa, rank, spec, dtype):
+    dX = x2.new_empty(x2.shape, dtype=torch.bfloat16)
+    if spec:
+        return dX, x2.new_empty((max(hip_ops.unpack_layout(spec)[1], 1),), dtype=dtype)
+    return dX, _grads_fake(x2, hip_ops.lora_qkv_grad_shapes(x2.shape[1],
+                                                            [d.shape[1] for d in dys], rank))
+
+
 # The LoRA backwards return (dX, grads): grads is one fp32 buffer holding the
 # adapter gradients as laid out by hip_ops.grad_layout (hip_ops.grad_views
 # splits it), so that the caller can cast them to the parameters' dtype in

@@ -10,7 +10,8 @@
 //     (see "256 x 256" below): the FLCE dW product, the FLCE products of a
 //     repeated (retain_graph) backward and the products with an MN-major A;
 //   - r4: 4 waves of 128 x 128, k-tiles of 64, five 32 KB operand slots
-//     (see "r4" below):
+//     (see "r4" below; also with a 128 x 128 tile, 4 waves of 64 x 64, for
+//     products with too few 256 x 256 tiles: see "choice of the tile"):
 //     the products with a K-major A (LoRA forward / dX / dH, the FLCE logits
 //     and dH products, the plain GEMM entry points).
 // Narrow tiles Cfg<BM, BN, WAVES_M> (256 x 32, 64 x 256: the rank-r LoRA
@@ -30,8 +31,8 @@
 //   pointers and leading dimensions (e.g. [dQ | dK | dV | lora] against
 //   [Wq; Wk; Wv; A]); a segment's last k-tile is zero-filled past its end.
 // Split-K
-//   with ksplit > 1 (single segment), split s accumulates the 64-wide
-//   k-tiles [s * kps, (s + 1) * kps) and the epilogue receives s;
+//   with ksplit > 1 (a single segment, on r4 any), split s accumulates the
+//   64-wide k-tiles [s * kps, (s + 1) * kps) and the epilogue receives s;
 //   EpiPartial writes fp32 partial tiles that reduce_partials_kernel sums in
 //   a fixed order.
 // Tile order

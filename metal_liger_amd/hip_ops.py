@@ -993,25 +993,46 @@ def lora_qkv_out(x2: torch.Tensor, ws, xa: torch.Tensor, sbs) -> list:
     x2, xa = _al16(x2, xa)
     ws = [_al16(w) for w in ws]
     sbs = [_al16(sb) for sb in sbs]
+    return _lora_outs(x2, ws, xa, [sb.data_ptr() for sb in sbs], [sb.stride(0) for sb in sbs],
+                      sbs[0].shape[1])
+
+
+def _lora_outs(x2, ws, xa, sb_ptrs, sb_strides, rp: int) -> list:
     N, K = x2.shape
-    rp = sbs[0].shape[1]
+    n = len(ws)
     outs = [torch.empty(N, w.shape[0], dtype=torch.bfloat16, device=x2.device) for w in ws]
     if N == 0:
         return outs
-    k_lens, a_p, ldas, b_p, ldbs = [], [], [], [], []
-    for i, (w, sb) in enumerate(zip(ws, sbs)):
-        k_lens += [K, rp]
-        a_p += [x2.data_ptr(), xa.data_ptr() + i * rp * xa.element_size()]
-        ldas += [x2.stride(0), xa.stride(0)]
-        b_p += [w.data_ptr(), sb.data_ptr()]
-        ldbs += [w.stride(0), sb.stride(0)]
+    xp, xap, xs, xas = x2.data_ptr(), xa.data_ptr(), x2.stride(0), xa.stride(0)
+    a_p, b_p, ldbs = [], [], []
+    for i, w in enumerate(ws):
+        a_p += (xp, xap + 2 * i * rp)
+        b_p += (w.data_ptr(), sb_ptrs[i])
+        ldbs += (w.stride(0), sb_strides[i])
+    widths = geom([w.shape[0] for w in ws])
     call(
-        "ml_gemm_bf16_segments_group", len(ws), geom([N] * len(ws)), geom([w.shape[0] for w in ws]),
-        _hip.ints([2] * len(ws)), geom(k_lens), _hip.ptrs(a_p), geom(ldas), _hip.ptrs(b_p),
-        geom(ldbs), 0, _hip.ptrs([o.data_ptr() for o in outs]), geom([o.stride(0) for o in outs]),
-        _hip.BF16, 1.0, 0.0, stream_of(x2),
+        "ml_gemm_bf16_segments_group", n, geom([N] * n), widths, _hip.ints([2] * n),
+        geom([K, rp] * n), _hip.ptrs(a_p), geom([xs, xas] * n), _hip.ptrs(b_p), geom(ldbs), 0,
+        _hip.ptrs([o.data_ptr() for o in outs]), widths, _hip.BF16, 1.0, 0.0, stream_of(x2),
     )
     return outs
+
+
+def lora_qkv_fwd(x2: torch.Tensor, ws, As, Bs, scales, rank: int):
+    """The q, k, v LoRA projections of x2 from the adapters as they are: the
+    pack, X A^T and the three products in one call. Returns (outs, X A^T [N,
+    3 rank], the packed adapters)."""
+    x2 = _al16(x2)
+    ws = [_al16(w) for w in ws]
+    packed = lora_pack(As, Bs, scales, rank)
+    n, base = len(As), packed.data_ptr()
+    xa = lora_xa(x2, packed[:n * rank * x2.shape[1]].view(n * rank, x2.shape[1]))
+    at = base + 2 * rank * (n * x2.shape[1] + sum(b.shape[0] for b in Bs))
+    sbs = []
+    for b in Bs:
+        sbs.append(at)
+        at += 2 * rank * b.shape[0]
+    return _lora_outs(x2, ws, xa, sbs, [rank] * n, rank), xa, packed
 
 
 # The adapter gradients of one LoRA backward call live in one fp32 buffer:
@@ -1056,24 +1077,45 @@ def lora_qkv_bwd(x2, dys, ws_, a_stack, bs, scales, xa, rank):
     """Returns (dX bf16 [N, in], grads fp32): grads holds dA [3r, in] and
     dB_i [out_i, r] as laid out by grad_layout(lora_qkv_grad_shapes(...))."""
     ensure_rocm_device(x2, *dys, *ws_, a_stack, *bs, xa)
-    x2, a_stack, xa = _dense16(x2, a_stack, xa)
-    dys, ws_, bs = [list(_dense16(*t, None))[:-1] for t in (dys, ws_, bs)]
+    a_stack, bs = _dense16(a_stack), list(_dense16(*bs, None))[:-1]
+    return _lora_qkv_bwd(x2, dys, ws_, a_stack.data_ptr(), [b.data_ptr() for b in bs], scales, xa,
+                         rank)
+
+
+def _lora_qkv_bwd(x2, dys, ws_, a_ptr, b_ptrs, scales, xa, rank):
+    x2, xa = _dense16(x2, xa)
+    dys, ws_ = [list(_dense16(*t, None))[:-1] for t in (dys, ws_)]
     N, IN = x2.shape
     outs = [int(d.shape[1]) for d in dys]
     dev = x2.device
     dX = torch.empty(N, IN, dtype=torch.bfloat16, device=dev)
-    flat, (dA, *dBs) = _grad_buffer(lora_qkv_grad_shapes(IN, outs, rank), dev)
+    offs, total = grad_layout(lora_qkv_grad_shapes(IN, outs, rank))
+    flat = torch.empty(max(total, 1), dtype=torch.float32, device=dev)
     if N == 0:   # no tokens: the adapter gradients are empty sums
         return dX, flat.zero_()
-    wsb = _hip.query("ml_lora_qkv_bwd_workspace_bytes", N, IN, geom(outs), rank)
+    out_geom, g = geom(outs), flat.data_ptr()
+    wsb = _hip.query("ml_lora_qkv_bwd_workspace_bytes", N, IN, out_geom, rank)
     ws = torch.empty(max(wsb, 16), dtype=torch.uint8, device=dev)
     call(
-        "ml_lora_qkv_bwd", ptr(x2), N, IN, _hip.ptrs([d.data_ptr() for d in dys]), geom(outs),
-        _hip.ptrs([w.data_ptr() for w in ws_]), ptr(a_stack), _hip.ptrs([b.data_ptr() for b in bs]),
-        _hip.floats(scales), ptr(xa), rank, ptr(dX), ptr(dA),
-        _hip.ptrs([b.data_ptr() for b in dBs]), ptr(ws), ws.numel(), stream_of(x2),
+        "ml_lora_qkv_bwd", x2.data_ptr(), N, IN, _hip.ptrs([d.data_ptr() for d in dys]), out_geom,
+        _hip.ptrs([w.data_ptr() for w in ws_]), a_ptr, _hip.ptrs(b_ptrs), _hip.floats(scales),
+        xa.data_ptr(), rank, dX.data_ptr(), g + 4 * offs[0],
+        _hip.ptrs([g + 4 * o for o in offs[1:]]), ws.data_ptr(), ws.numel(), stream_of(x2),
     )
     return dX, flat
+
+
+def lora_qkv_bwd_packed(x2, dys, ws_, packed, scales, xa, rank, spec, dtype):
+    """lora_qkv_bwd with the adapters as lora_qkv_fwd packed them; spec not
+    empty: the gradients as lora_unpack(grads, spec, dtype)."""
+    ensure_rocm_device(x2, *dys, *ws_, packed, xa)
+    base = packed.data_ptr()
+    at, b_ptrs = base + 2 * rank * len(dys) * x2.shape[1], []
+    for d in dys:
+        b_ptrs.append(at)
+        at += 2 * rank * d.shape[1]
+    dX, flat = _lora_qkv_bwd(x2, dys, ws_, base, b_ptrs, scales, xa, rank)
+    return dX, lora_unpack(flat, spec, dtype) if spec else flat
 
 
 def lora_linear_grad_shapes(IN, OUT, rank):

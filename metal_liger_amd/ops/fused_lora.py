@@ -146,20 +146,32 @@ def _adapter_grads(flat, shapes, parts, dtypes):
     row, rows, cols) of each. When the adapters share a dtype, one launch
     brings all of them to it and to dense matrices without the ranks' padding,
     instead of autograd casting each gradient in a launch of its own."""
+    spec, unpack = _grad_spec(shapes, parts, dtypes)
+    if unpack and flat.is_cuda:
+        return _unpacked_views(_ops.lora_unpack(flat, spec, dtypes[0]), spec)
+    return _grad_views(flat.to(dtypes[0]) if unpack else flat, spec)
+
+
+def _grad_spec(shapes, parts, dtypes):
+    """(lora_unpack's spec of the gradients, whether it is needed)."""
     offs, _ = hip_ops.grad_layout(shapes)
-    spec = []
+    spec, padded = [], False
     for k, row, rows, cols in parts:
         ld = shapes[k][1]
+        padded = padded or cols != ld
         spec += (offs[k] + row * ld, rows, cols, ld)
-    groups = [spec[i:i + 4] for i in range(0, len(spec), 4)]
-    if len(set(dtypes)) == 1 and dtypes[0] in (torch.float32, torch.bfloat16, torch.float16) and (
-            dtypes[0] != flat.dtype or any(cols != ld for _, _, cols, ld in groups)):
-        if flat.is_cuda:
-            flat = _ops.lora_unpack(flat, spec, dtypes[0])
-            at, _ = hip_ops.unpack_layout(spec)
-            return [_view(flat, (o, rows, cols)) for o, (_, rows, cols, _) in zip(at, groups)]
-        flat = flat.to(dtypes[0])
-    return [flat.as_strided((rows, cols), (ld, 1), off) for off, rows, cols, ld in groups]
+    same = len(set(dtypes)) == 1 and dtypes[0] in (torch.float32, torch.bfloat16, torch.float16)
+    return spec, same and (padded or dtypes[0] != torch.float32)
+
+
+def _grad_views(flat, spec):
+    return [flat.as_strided((spec[i + 1], spec[i + 2]), (spec[i + 3], 1), spec[i])
+            for i in range(0, len(spec), 4)]
+
+
+def _unpacked_views(flat, spec):
+    at, _ = hip_ops.unpack_layout(spec)
+    return [_view(flat, (o, spec[4 * i + 1], spec[4 * i + 2])) for i, o in enumerate(at)]
 
 
 def _lora_linear(X: torch.Tensor, W: torch.Tensor,
@@ -222,14 +234,12 @@ class _LoRA_QKV(torch.autograd.Function):
         ranks = [A.shape[0] for A in (QA, KA, VA)]
         rp = _pad_rank(max(ranks))
         scales = [float(QS), float(KS), float(VS)]
-        flat, a_views, Bs, sbs = _packed([QA, KA, VA], [QB, KB, VB], scales, rp)
-        a_stack = _stack_view(flat, a_views)
-        xa = cops.lora_xa(Xf, a_stack)                         # [N, 3 rp], saved
         Ws = [hip_ops._bf16_rows(W.detach()) for W in (QW, KW, VW)]
-        # the three projections in one launch: k and v alone would each leave
-        # half of the GPU idle for a round of tiles
-        outs = cops.lora_qkv_out(Xf, Ws, xa, sbs)
-        ctx.save_for_backward(Xf, xa, a_stack, *Ws, *Bs)
+        # one op: the packed adapters, X A^T [N, 3 rp] (both saved) and the three
+        # projections in one launch (k and v alone would each leave half of the
+        # GPU idle for a round of tiles)
+        *outs, xa, packed = cops.lora_qkv_fwd(Xf, Ws, [QA, KA, VA], [QB, KB, VB], scales, rp)
+        ctx.save_for_backward(Xf, xa, packed, *Ws)
         ctx.scales = scales
         ctx.ranks, ctx.rank_p = ranks, rp
         ctx.orig_shape = shape
@@ -254,16 +264,19 @@ class _LoRA_QKV(torch.autograd.Function):
                     None, grads[0][0], grads[0][1], None,
                     None, grads[1][0], grads[1][1], None,
                     None, grads[2][0], grads[2][1], None)
-        Xf, xa, a_stack, QW, KW, VW, QB, KB, VB = ctx.saved_tensors
+        Xf, xa, packed, QW, KW, VW = ctx.saved_tensors
         ranks, rp = ctx.ranks, ctx.rank_p
         shape = ctx.orig_shape
         dys = [hip_ops._bf16_rows(d.reshape(-1, d.shape[-1])) for d in (dQ, dK, dV)]
-        dX, flat = cops.lora_qkv_bwd(Xf, dys, [QW, KW, VW], a_stack, [QB, KB, VB],
-                                     ctx.scales, xa, rp)
         shapes = hip_ops.lora_qkv_grad_shapes(Xf.shape[1], [d.shape[1] for d in dys], rp)
         parts = [(0, i * rp, r, Xf.shape[1]) for i, r in enumerate(ranks)]
         parts += [(1 + i, 0, dys[i].shape[1], r) for i, r in enumerate(ranks)]
-        g = _adapter_grads(flat, shapes, parts, [t for pair in ctx.param_dtypes for t in pair])
+        dtypes = [t for pair in ctx.param_dtypes for t in pair]
+        spec, unpack = _grad_spec(shapes, parts, dtypes)
+        dX, flat = cops.lora_qkv_bwd_packed(Xf, dys, [QW, KW, VW], packed, ctx.scales, xa, rp,
+                                            spec if unpack else [],
+                                            dtypes[0] if unpack else torch.float32)
+        g = _unpacked_views(flat, spec) if unpack else _grad_views(flat, spec)
         grads = list(zip(g[:3], g[3:]))
         dX = dX.view(*shape)
         return (dX,

@@ -80,3 +80,27 @@ def test_backward_at_every_rank(n, rank, adapter):
             assert rel_fro(g, w) <= 2e-2, (fn.__name__, tuple(g.shape), float(rel_fro(g, w)))
         for g, leaf in zip(grads, leaves):
             assert g.dtype == leaf.dtype and g.is_contiguous()
+
+
+def test_fake_kernels_match():
+    import metal_liger_amd._custom_ops  # noqa: F401
+    ops = torch.ops.metal_liger_amd
+    check = ("test_schema", "test_faketensor")
+    x = seeded((40, 64), 1, BF).cuda()
+    Ws = [seeded((o, 64), 2 + o, BF).cuda() for o in (48, 24, 24)]
+    As = [seeded((5, 64), 3 + k, torch.float32).cuda() for k in range(3)]
+    Bs = [seeded((o, 5), 6 + o, torch.float32).cuda() for o in (48, 24, 24)]
+    scales, rank = [2.0, 2.0, 2.0], 16
+    torch.library.opcheck(ops.lora_pack.default, (As, Bs, scales, rank), test_utils=check)
+    torch.library.opcheck(ops.lora_qkv_fwd.default, (x, Ws, As, Bs, scales, rank), test_utils=check)
+    q, k, v, xa, packed = ops.lora_qkv_fwd(x, Ws, As, Bs, scales, rank)
+    spec = [0, 5, 64, 64, 3072, 48, 5, 16]
+    for sp in (spec, []):
+        torch.library.opcheck(ops.lora_qkv_bwd_packed.default,
+                              (x, [q, k, v], Ws, packed, scales, xa, rank, sp, torch.float32),
+                              test_utils=check)
+    torch.library.opcheck(ops.lora_unpack.default, (seeded((4000,), 7).cuda(), spec, BF),
+                          test_utils=check)
+    kv = [seeded((2, 4, 5, 16), 8 + i, BF).cuda() for i in range(2)]
+    torch.library.opcheck(ops.kv_expand.default, (*kv, 2), test_utils=check)
+    torch.library.opcheck(ops.kv_reduce.default, (*kv, 2), test_utils=check)
