@@ -222,15 +222,12 @@ __device__ __forceinline__ float grp16_reduce16(float (&x)[16], int c) {
 // into the hidden rows of the dW product instead of a pass over the [T, V]
 // buffer.
 // live: rows of the chunk past it are not computed.
-// tile_flags (optional): only row tiles with a nonzero flag are computed
-// (the recomputation of rows whose shift was out of range).
 constexpr int kShiftBlock = 128;  // columns per partial: one r4 wave's sub-tile
 
 template <typename TB>
 struct EpiShiftExp {
   const TB* bias;
   const float* shift;     // [M]
-  const int* tile_flags;  // null: every tile
   float* pmax;            // [M][nblk]
   float* psum;            // [M][nblk]
   bf16* E;
@@ -241,10 +238,6 @@ struct EpiShiftExp {
   using LiveM = void;
   __device__ __forceinline__ void live_m(const Problem&, int& tiles_m, int&, int&) const {
     tiles_m = (live.count() + 255) / 256;
-  }
-
-  __device__ __forceinline__ bool skip_tile(int tm) const {
-    return tile_flags != nullptr && tile_flags[tm] == 0;
   }
 
   // acc[h][i][j][v]: row m0 + 16 i + 4 (lane / 16) + v, column n0 + 64 h +
@@ -367,6 +360,26 @@ struct EpiShiftExp {
       tile<false>(acc, m0, n0, lane, lds);
   }
 };
+
+// The logits of the row tiles (blockIdx.y) that a row flagged, once more, the
+// column tiles shared out over blockIdx.x (one block per CU and row tile, so a
+// single flagged tile has the whole chip). Almost every launch finds no flag,
+// and what counts is how soon its blocks return.
+template <typename TB>
+__global__ __launch_bounds__(R4Cfg::THREADS) void recompute_kernel(
+    const Problem pb, const EpiShiftExp<TB> epi, const int* __restrict__ tile_flags) {
+  const int tm = blockIdx.y;
+  if (tile_flags[tm] == 0) return;
+  __shared__ __attribute__((aligned(16))) char lds[r4::Geom<8>::LDS_BYTES];
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  for (int tn = blockIdx.x; tn < pb.tiles_n; tn += gridDim.x) {
+    f32x4_t acc[2][r4::TM][4];
+    r4_mainloop<kKMajor, kKMajor, 8, false>(pb, tm, tn, 0, 1, 0, lds, acc);
+    epi.full_tile(acc, tm * 256 + (wave >> 1) * r4::WM, tn * 256 + (wave & 1) * r4::WN,
+                  threadIdx.x & 63, lds + wave * r4::Geom<8>::WAVE_EPI);
+    __syncthreads();  // the epilogue's LDS is the next tile's operand slots
+  }
+}
 
 // zy[t] = h_t . W[label_t] (+ b[label_t]) for a label in [0, V), else 0
 // (the label logit, as the reference forms it from the gathered weight rows,
@@ -1181,10 +1194,13 @@ int fwd_grad_impl(const bf16* hidden, int64_t ldh, const bf16* weight, int64_t l
     // then the same two steps again for the row tiles a row flagged (their
     // blocks alone do work; for the others the launches return at once)
     for (int pass = 0; pass < 2; ++pass) {
-      EpiShiftExp<TB> epi{bias, w.shift, pass ? w.tile_flags : nullptr, w.pmax, w.psum, w.E,
-                          (int64_t)V, Tc, V, nsb, live};
-      gemm_kernel<R4Cfg, kKMajor, kKMajor, EpiShiftExp<TB>>
-          <<<dim3(grid_blocks(pb)), R4Cfg::THREADS, 0, st>>>(pb, epi);
+      EpiShiftExp<TB> epi{bias, w.shift, w.pmax, w.psum, w.E, (int64_t)V, Tc, V, nsb, live};
+      if (pass == 0)
+        gemm_kernel<R4Cfg, kKMajor, kKMajor, EpiShiftExp<TB>>
+            <<<dim3(grid_blocks(pb)), R4Cfg::THREADS, 0, st>>>(pb, epi);
+      else
+        recompute_kernel<TB><<<dim3((unsigned)std::min(pb.tiles_n, kDhCUs), (unsigned)pb.tiles_m),
+                               R4Cfg::THREADS, 0, st>>>(pb, epi, w.tile_flags);
       ML_LAUNCH_CHECK();
       bf16* hs = d_weight ? w.Hs : nullptr;
       if (pass == 0)

@@ -1552,14 +1552,6 @@ __device__ __forceinline__ void load_row8_bf16(const bf16* p, int n, int N, floa
 //   (f32x4_t[8][4] for the 256 x 256 tile, f32x16_t[TM][TN] otherwise).
 //   smem: LDS the epilogue may use - for the 256 x 256 tile, 16 KB private
 //   to the wave (staged bf16 epilogues); otherwise the block's stage 0.
-// An epilogue may declare skip_tile(tm): work items of row tiles it skips
-// return before the main loop (a block-uniform test, no barrier reached).
-template <class E, class = void>
-struct HasSkipTile : std::false_type {};
-template <class E>
-struct HasSkipTile<E, std::void_t<decltype(std::declval<const E&>().skip_tile(0))>>
-    : std::true_type {};
-
 // An epilogue of the r4 engine may take a wave's whole 128 x 128 sub-tile in
 // one call: full_tile(acc, m0, n0, lane, lds) with acc[h][i][j] the MFMA
 // tile (i, 4 h + j) and lds the wave's 2 x 16 KB; otherwise it is called per
@@ -1596,9 +1588,6 @@ __global__ __launch_bounds__(C::THREADS) void gemm_kernel(const Problem pb, cons
   int tiles_m = pb.tiles_m, ksplit = pb.ksplit, kps = pb.kps;
   if constexpr (HasLiveM<Epi>::value) epi.live_m(pb, tiles_m, ksplit, kps);
   if (!tile_coords(pb, tiles_m, ksplit, blockIdx.x, tm, tn, split)) return;
-  if constexpr (HasSkipTile<Epi>::value) {
-    if (epi.skip_tile(tm)) return;
-  }
   const int tid = threadIdx.x;
   const int wave = tid >> 6;
   if constexpr (C::ENGINE == 2) {
