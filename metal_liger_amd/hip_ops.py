@@ -1022,6 +1022,7 @@ def lora_qkv_fwd(x2: torch.Tensor, ws, As, Bs, scales, rank: int):
     """The q, k, v LoRA projections of x2 from the adapters as they are: the
     pack, X A^T and the three products in one call. Returns (outs, X A^T [N,
     3 rank], the packed adapters)."""
+    ensure_rocm_device(x2, *ws, *As, *Bs)
     x2 = _al16(x2)
     ws = [_al16(w) for w in ws]
     packed = lora_pack(As, Bs, scales, rank)

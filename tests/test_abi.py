@@ -102,3 +102,11 @@ def test_flce_dh_split_count_fills_its_rounds():
         items = -(-T // 256) * (H // 256) * splits
         rounds = -(-items // 256)
         assert rounds == 1 or items - (rounds - 1) * 256 >= 192, (T, splits, items)
+
+
+def test_launches_refuse_cpu_tensors():
+    """Every launch asks for its tensor's stream: a CPU tensor is refused there
+    too, whatever the wrapper checked."""
+    import torch
+    with pytest.raises(ValueError, match="ROCm GPU"):
+        _hip.stream_of(torch.empty(1))
