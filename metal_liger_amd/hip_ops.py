@@ -889,6 +889,18 @@ def _ksplit_for(tiles: int, k: int) -> int:
     return max(1, min(ktiles, (512 + tiles - 1) // max(tiles, 1)))
 
 
+def check_adapters(ins, ws, As, Bs) -> None:
+    """Projection i maps ins[i] features by W_i [out_i, in_i] and the adapter A_i
+    [r_i, in_i], B_i [out_i, r_i]. The packed adapters are read at offsets that
+    follow from W's sizes, and the kernels take no sizes from the tensors: a
+    mismatch would read the neighbouring matrix, or past the buffer."""
+    for i, (n, w, a, b) in enumerate(zip(ins, ws, As, Bs)):
+        if w.dim() != 2 or a.dim() != 2 or b.dim() != 2 or not (
+                w.shape[1] == a.shape[1] == n and b.shape[0] == w.shape[0]):
+            raise ValueError(f"LoRA projection {i}: adapter A {tuple(a.shape)}, B {tuple(b.shape)} "
+                             f"and weight {tuple(w.shape)} do not fit {n} input features")
+
+
 def lora_pack(As, Bs, scales, rank: int) -> torch.Tensor:
     """The adapters' parameters in bf16 with ranks padded by zeros to `rank`,
     in one buffer and one launch: every A_i [rank, in_i], then every B_i
@@ -946,6 +958,8 @@ def lora_xa(x2: torch.Tensor, a_stack: torch.Tensor) -> torch.Tensor:
     256x32 tiles, split-K over in."""
     N, K = x2.shape
     R = a_stack.shape[0]
+    if a_stack.shape[1] != K:
+        raise ValueError(f"lora_xa: adapter {tuple(a_stack.shape)} does not fit {K} input features")
     if R <= 192 and K % 8 == 0 and x2.stride(-1) == 1 and x2.stride(0) % 8 == 0:
         out = torch.empty(N, R, dtype=torch.bfloat16, device=x2.device)
         if N == 0:
@@ -1022,6 +1036,7 @@ def lora_qkv_fwd(x2: torch.Tensor, ws, As, Bs, scales, rank: int):
     """The q, k, v LoRA projections of x2 from the adapters as they are: the
     pack, X A^T and the three products in one call. Returns (outs, X A^T [N,
     3 rank], the packed adapters)."""
+    check_adapters([x2.shape[1]] * len(ws), ws, As, Bs)
     ensure_rocm_device(x2, *ws, *As, *Bs)
     x2 = _al16(x2)
     ws = [_al16(w) for w in ws]

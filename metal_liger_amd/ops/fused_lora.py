@@ -107,10 +107,12 @@ def _pad_rank(r: int) -> int:
     return (r + 15) // 16 * 16 if r <= 64 else (r + 7) // 8 * 8
 
 
-def _packed(As, Bs, scales, rp: int):
-    """The adapters in bf16, ranks padded with zeros to rp: (buffer, where each
-    A_i lies in it, [B_i], [s_i B_i]). One buffer, formed in one launch; tensors that are not on a GPU (the products
-    refuse them) are formed by torch."""
+def _packed(ins, Ws, As, Bs, scales, rp: int):
+    """The adapters of projections from ins[i] features by W_i, in bf16, ranks
+    padded with zeros to rp: (buffer, where each A_i lies in it, [B_i], [s_i
+    B_i]). One buffer, formed in one launch; tensors that are not on a GPU (the
+    products refuse them) are formed by torch."""
+    hip_ops.check_adapters(ins, Ws, As, Bs)
     n = len(As)
     if As[0].is_cuda:
         flat = _ops.lora_pack(list(As), list(Bs), scales, rp)
@@ -193,7 +195,8 @@ def _lora_linear(X: torch.Tensor, W: torch.Tensor,
     if A is None or B is None:
         out = cops.linear_bf16(X2, W2)
     else:
-        flat, a_views, _, (sb,) = _packed([A], [B], [float(scaling)], _pad_rank(A.shape[0]))
+        flat, a_views, _, (sb,) = _packed([shape[-1]], [W], [A], [B], [float(scaling)],
+                                           _pad_rank(A.shape[0]))
         xa = cops.lora_xa(X2, _stack_view(flat, a_views))
         out = cops.lora_linear_out(X2, W2, xa, sb)
     return out.view(*shape[:-1], out.shape[-1])
@@ -312,7 +315,8 @@ class _LoRA_MLP(torch.autograd.Function):
         ranks = [A.shape[0] for A in (GA, UA, DA)]  # padded to the largest, as in _LoRA_QKV
         rp = _pad_rank(max(ranks))
         scales = [float(GS), float(US), float(DS)]
-        flat, a_views, (BG, BU, BD), (sG, sU, sD) = _packed([GA, UA, DA], [GB, UB, DB], scales, rp)
+        flat, a_views, (BG, BU, BD), (sG, sU, sD) = _packed(
+            [shape[-1], shape[-1], GW.shape[0]], [GW, UW, DW], [GA, UA, DA], [GB, UB, DB], scales, rp)
         a_gu = _stack_view(flat, a_views[:2])                    # [2 rp, hidden]
         a_d = _stack_view(flat, a_views[2:])                     # [rp, inter]
         GWc, UWc, DWc = (hip_ops._bf16_rows(W.detach()) for W in (GW, UW, DW))
@@ -390,7 +394,7 @@ class _LoRA_W(torch.autograd.Function):
         r = A.shape[0]
         rp = _pad_rank(r)
         scale = float(S)
-        flat, a_views, (Bp,), (sb,) = _packed([A], [B], [scale], rp)
+        flat, a_views, (Bp,), (sb,) = _packed([shape[-1]], [W], [A], [B], [scale], rp)
         a = _stack_view(flat, a_views)
         xa = cops.lora_xa(Xf, a)                                 # [N, rp], saved
         Wc = hip_ops._bf16_rows(W.detach())
