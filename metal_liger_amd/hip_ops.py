@@ -893,10 +893,12 @@ def check_adapters(ins, ws, As, Bs) -> None:
     """Projection i maps ins[i] features by W_i [out_i, in_i] and the adapter A_i
     [r_i, in_i], B_i [out_i, r_i]. The packed adapters are read at offsets that
     follow from W's sizes, and the kernels take no sizes from the tensors: a
-    mismatch would read the neighbouring matrix, or past the buffer."""
+    mismatch would read the neighbouring matrix, or past the buffer, and ranks
+    that differ would be padded to one."""
     for i, (n, w, a, b) in enumerate(zip(ins, ws, As, Bs)):
         if w.dim() != 2 or a.dim() != 2 or b.dim() != 2 or not (
-                w.shape[1] == a.shape[1] == n and b.shape[0] == w.shape[0]):
+                w.shape[1] == a.shape[1] == n and b.shape[0] == w.shape[0]
+                and a.shape[0] == b.shape[1]):
             raise ValueError(f"LoRA projection {i}: adapter A {tuple(a.shape)}, B {tuple(b.shape)} "
                              f"and weight {tuple(w.shape)} do not fit {n} input features")
 

@@ -17,8 +17,10 @@ def _projection(i, o, r=8, a=None, b=None):
             torch.zeros(b or (o, r), dtype=BF), 2.0]
 
 
-# what is wrong with the one adapter: A narrower, A wider, B shorter, B longer
-WRONG = [dict(a=(8, 56)), dict(a=(8, 72)), dict(b=(24, 8)), dict(b=(40, 8))]
+# what is wrong with the one adapter: A narrower, A wider, B shorter, B longer,
+# a B of more or less than A's rank (within the rank that the kernels pad to)
+WRONG = [dict(a=(8, 56)), dict(a=(8, 72)), dict(b=(24, 8)), dict(b=(40, 8)), dict(b=(32, 12)),
+         dict(b=(32, 4))]
 
 
 def _args(projections, wrong, at):
@@ -34,7 +36,7 @@ def test_blocks_refuse_adapters_that_do_not_fit(at, wrong):
         _LoRA_QKV.apply(x, *_args([(64, 32)] * 3, wrong, at))
     inter = [(64, 32), (64, 32), (32, 64)]
     if at == 2:   # the down projection's sizes are the other way round
-        wrong = {k: (v[1], v[0]) if k == "a" else (v[0] + 32, v[1]) for k, v in wrong.items()}
+        wrong = {k: (8, v[1] - 32) if k == "a" else (v[0] + 32, v[1]) for k, v in wrong.items()}
     with pytest.raises(ValueError, match="do not fit (64|32) input features"):
         _LoRA_MLP.apply(x, *_args(inter, wrong, at))
 
