@@ -962,6 +962,7 @@ def lora_xa(x2: torch.Tensor, a_stack: torch.Tensor) -> torch.Tensor:
     R = a_stack.shape[0]
     if a_stack.shape[1] != K:
         raise ValueError(f"lora_xa: adapter {tuple(a_stack.shape)} does not fit {K} input features")
+    ensure_rocm_device(x2, a_stack)
     if R <= 192 and K % 8 == 0 and x2.stride(-1) == 1 and x2.stride(0) % 8 == 0:
         out = torch.empty(N, R, dtype=torch.bfloat16, device=x2.device)
         if N == 0:
@@ -983,6 +984,7 @@ def _segments_ws_bytes(M: int, N: int, *k_lens: int) -> int:
 def lora_linear_out(x2: torch.Tensor, w: torch.Tensor, xa: torch.Tensor,
                     sb: torch.Tensor) -> torch.Tensor:
     """X W^T + XA (s B)^T as ONE K-concatenated GEMM -> [N, out] bf16."""
+    ensure_rocm_device(x2, w, xa, sb)
     x2, w, xa, sb = _al16(x2, w, xa, sb)
     N, K = x2.shape
     out_f = w.shape[0]
@@ -1006,6 +1008,7 @@ def lora_qkv_out(x2: torch.Tensor, ws, xa: torch.Tensor, sbs) -> list:
     """The q, k, v LoRA projections X W_i^T + XA_i (s_i B_i)^T (XA_i the i-th
     block of rank columns of xa) as three K-concatenated products in ONE
     grouped launch -> three [N, out_i] bf16 tensors."""
+    ensure_rocm_device(x2, *ws, xa, *sbs)
     x2, xa = _al16(x2, xa)
     ws = [_al16(w) for w in ws]
     sbs = [_al16(sb) for sb in sbs]

@@ -61,3 +61,41 @@ def test_weights_that_do_not_fit_the_input_are_refused():
 def test_stacked_adapters_of_another_width_are_refused(rows):
     with pytest.raises(ValueError, match="does not fit 64 input features"):
         hip_ops.lora_xa(torch.zeros(4, 64, dtype=BF), torch.zeros(rows, 72, dtype=BF))
+
+
+def _seen_by_the_device_check(monkeypatch, fn, *args):
+    """The tensors that fn checks for being on one GPU before it launches."""
+    class Checked(Exception):
+        pass
+
+    def check(*tensors):
+        raise Checked(tensors)
+
+    monkeypatch.setattr(hip_ops, "ensure_rocm_device", check)
+    with pytest.raises(Checked) as e:
+        fn(*args)
+    return {id(t) for t in e.value.args[0]}
+
+
+def test_every_operand_of_the_products_is_checked_for_its_device(monkeypatch):
+    """An adapter left on the CPU beside an input on the GPU must not reach a
+    kernel as a host pointer."""
+    x, w, a, xa, sb = (torch.zeros(s, dtype=BF)
+                       for s in ((4, 64), (32, 64), (16, 64), (4, 16), (32, 16)))
+    seen = _seen_by_the_device_check(monkeypatch, hip_ops.lora_xa, x, a)
+    assert {id(x), id(a)} <= seen
+    seen = _seen_by_the_device_check(monkeypatch, hip_ops.lora_linear_out, x, w, xa, sb)
+    assert {id(t) for t in (x, w, xa, sb)} <= seen
+    seen = _seen_by_the_device_check(monkeypatch, hip_ops.lora_qkv_out, x, [w] * 3, xa, [sb] * 3)
+    assert {id(t) for t in (x, w, xa, sb)} <= seen
+
+
+@pytest.mark.gpu
+def test_adapters_on_another_device_are_refused(dev):
+    x = torch.zeros(4, 64, dtype=BF, device=dev)
+    one = _projection(64, 32)
+    for fn in (_LoRA_W.apply, _lora_linear):
+        for on_gpu in range(7):   # every subset of the weight, A and B but all of them
+            args = [t.to(dev) if on_gpu >> k & 1 else t for k, t in enumerate(one[:3])]
+            with pytest.raises((ValueError, RuntimeError), match="ROCm GPU|device"):
+                fn(x, *args, 2.0)
