@@ -115,7 +115,7 @@ def _packed(ins, Ws, As, Bs, scales, rp: int):
     hip_ops.check_adapters(ins, Ws, As, Bs)
     n = len(As)
     if As[0].is_cuda:
-        flat = _ops.lora_pack(list(As), list(Bs), scales, rp)
+        flat = _ops.lora_pack([A.detach() for A in As], [B.detach() for B in Bs], scales, rp)
     else:
         pad = nn.functional.pad
         a = [pad(A.detach().to(torch.bfloat16), (0, 0, 0, rp - A.shape[0])) for A in As]

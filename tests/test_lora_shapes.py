@@ -99,3 +99,14 @@ def test_adapters_on_another_device_are_refused(dev):
             args = [t.to(dev) if on_gpu >> k & 1 else t for k, t in enumerate(one[:3])]
             with pytest.raises((ValueError, RuntimeError), match="ROCm GPU|device"):
                 fn(x, *args, 2.0)
+
+
+def test_plain_projection_does_not_ask_for_adapter_gradients():
+    """_lora_linear records nothing for its adapters (the Functions do): its
+    result must not require a gradient that cannot be formed."""
+    from torch._subclasses.fake_tensor import FakeTensorMode
+    with FakeTensorMode():
+        x, w, a, b = (torch.empty(s, dtype=BF, device="cuda:0")
+                      for s in ((4, 64), (32, 64), (8, 64), (32, 8)))
+        out = _lora_linear(x, w, a.requires_grad_(), b.requires_grad_(), 2.0)
+    assert out.shape == (4, 32) and not out.requires_grad
