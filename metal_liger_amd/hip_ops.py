@@ -896,11 +896,11 @@ def check_adapters(ins, ws, As, Bs) -> None:
     mismatch would read the neighbouring matrix, or past the buffer, and ranks
     that differ would be padded to one."""
     for i, (n, w, a, b) in enumerate(zip(ins, ws, As, Bs)):
-        if w.dim() != 2 or a.dim() != 2 or b.dim() != 2 or not (
-                w.shape[1] == a.shape[1] == n and b.shape[0] == w.shape[0]
-                and a.shape[0] == b.shape[1]):
-            raise ValueError(f"LoRA projection {i}: adapter A {tuple(a.shape)}, B {tuple(b.shape)} "
-                             f"and weight {tuple(w.shape)} do not fit {n} input features")
+        w, a, b = w.shape, a.shape, b.shape
+        if not (len(w) == len(a) == len(b) == 2 and w[1] == a[1] == n and b[0] == w[0]
+                and a[0] == b[1]):
+            raise ValueError(f"LoRA projection {i}: adapter A {tuple(a)}, B {tuple(b)} and weight "
+                             f"{tuple(w)} do not fit {n} input features")
 
 
 def lora_pack(As, Bs, scales, rank: int) -> torch.Tensor:

@@ -35,7 +35,6 @@ import logging
 import torch
 import torch.nn as nn
 
-from metal_liger_amd import _custom_ops as _ops
 from metal_liger_amd import _custom_ops as cops
 from metal_liger_amd import hip_ops
 from metal_liger_amd._model_walk import find_layers, shadowed
@@ -115,7 +114,9 @@ def _packed(ins, Ws, As, Bs, scales, rp: int):
     hip_ops.check_adapters(ins, Ws, As, Bs)
     n = len(As)
     if As[0].is_cuda:
-        flat = _ops.lora_pack([A.detach() for A in As], [B.detach() for B in Bs], scales, rp)
+        if torch.is_grad_enabled():  # the plain projection; the Functions run without
+            As, Bs = [A.detach() for A in As], [B.detach() for B in Bs]
+        flat = cops.lora_pack(list(As), list(Bs), scales, rp)
     else:
         pad = nn.functional.pad
         a = [pad(A.detach().to(torch.bfloat16), (0, 0, 0, rp - A.shape[0])) for A in As]
@@ -150,7 +151,7 @@ def _adapter_grads(flat, shapes, parts, dtypes):
     instead of autograd casting each gradient in a launch of its own."""
     spec, unpack = _grad_spec(shapes, parts, dtypes)
     if unpack and flat.is_cuda:
-        return _unpacked_views(_ops.lora_unpack(flat, spec, dtypes[0]), spec)
+        return _unpacked_views(cops.lora_unpack(flat, spec, dtypes[0]), spec)
     return _grad_views(flat.to(dtypes[0]) if unpack else flat, spec)
 
 
