@@ -4,15 +4,18 @@
 // Two schedules share the kernels below.
 //
 // Loss and gradients in one pass (ml_flce_fwd_grad), over chunks of T tokens:
-//   0. the tokens' order (token_order_kernel): in the masked form
-//      (ml_flce_fwd_grad_masked) the tokens to be computed first and those with
+//   0. in the masked form (ml_flce_fwd_grad_masked) the tokens' order
+//      (token_order_kernel): the tokens to be computed first and those with
 //      the ignored label, whose gradients are zero, behind them. Every later
 //      step reads from the device how many rows of its chunk are live: row
 //      tiles past them return at once, the dH product splits the vocabulary
 //      over the workgroups this frees, and dW's K ends with them. [1000, 2048]
 //      x 151936 with 30% of the tokens ignored: 1.11 -> 0.85 ms;
-//   1. the chunk's rows gathered (bf16 [T, H]) with a shift per row, c = (label logit h . W[y], or the logit of entry 0
-//      for a row without a label in range) + 30 (shift_kernel);
+//      Without the mask only the labels are counted, and the rows stay where
+//      they are;
+//   1. a shift per row, c = (label logit h . W[y], or the logit of entry 0 for
+//      a row without a label in range) + 30, and in the masked form the chunk's
+//      rows gathered (bf16 [T, H]) (shift_kernel);
 //   2. Z = H_c W^T (+ b) as a bf16 MFMA GEMM whose epilogue stores e =
 //      exp(z - c) in bf16 ([T, vocab] buffer) and writes per-row, per
 //      64-column (max z, sum e) partials;
@@ -63,11 +66,15 @@ constexpr int kDhMaxSplit = 64;  // splits of the dH product
 constexpr int kColBlock = big::WN;  // columns per (max, sum) partial: one wave's sub-tile
 
 // The live rows of a chunk: positions t0 .. t0 + T - 1 of the tokens' order,
-// of which the first *n_live are computed.
+// of which the first *n_live are computed. Without the mask (both pointers null)
+// every token is, in place.
 struct LiveRows {
   const int* n_live;
+  const int* order;  // the chunk's part of it
   int t0, T;
+  __device__ __forceinline__ int token(int row) const { return order ? order[row] : t0 + row; }
   __device__ __forceinline__ int count() const {
+    if (n_live == nullptr) return T;
     const int n = __builtin_amdgcn_readfirstlane(*n_live) - t0;
     return n < 0 ? 0 : n < T ? n : T;
   }
@@ -446,12 +453,11 @@ __global__ __launch_bounds__(1024) void count_valid_kernel(const int64_t* __rest
 constexpr float kShiftMargin = 30.f;
 constexpr float kLogSMin = -36.f, kLogSMax = 48.f;
 
-// order: the tokens to be computed, then (masked) the ignored ones, each in
-// their own order; n_live = how many come first; n_valid = #(labels !=
-// ignore). Without masked every token is computed, in place. One block; a
-// thread takes 8 consecutive labels per step.
+// order: the tokens to be computed, then the ignored ones, each in their own
+// order; n_live = how many come first; n_valid = #(labels != ignore), the same
+// number. One block; a thread takes 8 consecutive labels per step.
 __global__ __launch_bounds__(1024) void token_order_kernel(const int64_t* __restrict__ labels,
-                                                           int N, int64_t ignore, bool masked,
+                                                           int N, int64_t ignore,
                                                            int* __restrict__ order,
                                                            int* __restrict__ n_live,
                                                            float* __restrict__ n_valid) {
@@ -480,11 +486,7 @@ __global__ __launch_bounds__(1024) void token_order_kernel(const int64_t* __rest
   const int valid = block_sum(wave_scan(c)).y;
   if (tid == 0) {
     n_valid[0] = (float)valid;
-    n_live[0] = masked ? valid : N;
-  }
-  if (!masked) {
-    for (int i = tid; i < N; i += 1024) order[i] = i;
-    return;
+    n_live[0] = valid;
   }
   int base = 0;  // valid tokens before this step's labels
   for (int64_t b = 0; b < N; b += 8192) {
@@ -508,33 +510,33 @@ __global__ __launch_bounds__(1024) void token_order_kernel(const int64_t* __rest
   }
 }
 
-// Row r of a chunk is token order[r] (the chunk's part of the order). Hc[r] =
-// the token's hidden row; zy[r] = h . W[label] (+ b) for a label in [0, V),
+// Row r of a chunk is token live.token(r). Hc[r] (unless Hc is null) = the
+// token's hidden row; zy[r] = h . W[label] (+ b) for a label in [0, V),
 // else 0; shift[r] = the pseudo-label logit + kShiftMargin. Block 0 also
 // clears the chunk's n_flags tile flags. One wave per live row; H % 8 == 0.
 template <typename TB>
 __global__ __launch_bounds__(256) void shift_kernel(
     const bf16* __restrict__ hidden, int64_t ldh, const bf16* __restrict__ weight, int64_t ldw,
-    const TB* __restrict__ bias, const int64_t* __restrict__ labels,
-    const int* __restrict__ order, const LiveRows live, int64_t V, int H, bf16* __restrict__ Hc,
-    float* __restrict__ zy, float* __restrict__ shift, int* __restrict__ tile_flags, int n_flags) {
+    const TB* __restrict__ bias, const int64_t* __restrict__ labels, const LiveRows live,
+    int64_t V, int H, bf16* __restrict__ Hc, float* __restrict__ zy, float* __restrict__ shift,
+    int* __restrict__ tile_flags, int n_flags) {
   if (blockIdx.x == 0)
     for (int i = threadIdx.x; i < n_flags; i += 256) tile_flags[i] = 0;
   const int lane = threadIdx.x & 63;
   const int row = blockIdx.x * 4 + (threadIdx.x >> 6);
   if (row >= live.count()) return;
-  const int64_t token = order[row];
+  const int64_t token = live.token(row);
   const int64_t lab = labels[token];
   const bool inrange = lab >= 0 && lab < V;
   const int64_t idx = inrange ? lab : 0;
   const bf16* h = hidden + token * ldh;
   const bf16* w = weight + idx * ldw;
-  bf16* hc = Hc + (int64_t)row * H;
+  bf16* hc = Hc ? Hc + (int64_t)row * H : nullptr;
   float acc = 0.f;
   for (int k = lane * 8; k < H; k += 64 * 8) {
     float a[8], b[8];
     load_n<bf16, 8>(h + k, a);
-    store_n<bf16, 8>(hc + k, a);
+    if (hc) store_n<bf16, 8>(hc + k, a);
     load_n<bf16, 8>(w + k, b);
 #pragma unroll
     for (int q = 0; q < 8; ++q) acc += a[q] * b[q];
@@ -555,7 +557,7 @@ __global__ __launch_bounds__(256) void shift_kernel(
 //   softmax * mask / #valid), the label entry rewritten as e' = exp(z_y - c)
 //   - S (alpha e' = (p_y - 1) * mask / #valid, from the fp32 label logit),
 //   and (Hs not null) the scaled hidden row Hs = alpha h (bf16; the dW
-//   product's operand).
+//   product's operand), h row `row` of rows.
 // A row outside the window (first pass) flags its tile and takes c = M. A row
 // past the live ones is an ignored token: loss term 0, lse = +inf (what a
 // repeated backward needs of it: exp(z - lse) = 0).
@@ -563,14 +565,14 @@ template <bool RECOMPUTE>
 __global__ __launch_bounds__(256) void finalize_kernel(
     const float* __restrict__ pmax, const float* __restrict__ psum, int nblk,
     float* __restrict__ shift, const float* __restrict__ zy, const int64_t* __restrict__ labels,
-    const int* __restrict__ order, const LiveRows live, int64_t ignore, int M, int64_t V,
-    const float* __restrict__ n_valid, bf16* __restrict__ E, int64_t ldE,
-    const bf16* __restrict__ Hc, int H, bf16* __restrict__ Hs, float* __restrict__ alpha, int* __restrict__ tile_flags, float* __restrict__ lse,
-    float* __restrict__ loss_row, float* __restrict__ valid_row) {
+    const LiveRows live, int64_t ignore, int M, int64_t V, const float* __restrict__ n_valid,
+    bf16* __restrict__ E, int64_t ldE, const bf16* __restrict__ rows, int64_t ldr, int H,
+    bf16* __restrict__ Hs, float* __restrict__ alpha, int* __restrict__ tile_flags,
+    float* __restrict__ lse, float* __restrict__ loss_row, float* __restrict__ valid_row) {
   const int lane = threadIdx.x & 63;
   const int row = blockIdx.x * 4 + (threadIdx.x >> 6);
   if (row >= M) return;
-  const int64_t token = order[row];
+  const int64_t token = live.token(row);
   if (row >= live.count()) {
     if (!RECOMPUTE && lane == 0) {
       lse[token] = INFINITY;
@@ -617,7 +619,7 @@ __global__ __launch_bounds__(256) void finalize_kernel(
     if (valid && inrange) E[(int64_t)row * ldE + lab] = from_f32<bf16>(exp_f(zy[row] - c) - s);
   }
   if (Hs == nullptr) return;
-  const bf16* h = Hc + (int64_t)row * H;
+  const bf16* h = rows + (int64_t)row * ldr;
   bf16* hs = Hs + (int64_t)row * H;
   for (int k = lane * 8; k < H; k += 64 * 8) {
     float x[8];
@@ -674,12 +676,11 @@ struct EpiDhPartial {
   }
 };
 
-// dH[order[r]] = alpha[r] * the sum of row r's partials in a fixed order for a
+// dH[live.token(r)] = alpha[r] * the sum of row r's partials in a fixed order for a
 // live row r, zeros for the others of the chunk. 8 columns per thread.
 __global__ __launch_bounds__(256) void dh_reduce_kernel(const float* __restrict__ P,
                                                         const DhSplits splits, const LiveRows live,
-                                                        const int* __restrict__ order, int M, int H,
-                                                        const float* __restrict__ alpha,
+                                                        int M, int H, const float* __restrict__ alpha,
                                                         bf16* __restrict__ dH) {
   const int rows = live.count();
   int ksplit, kps;
@@ -712,7 +713,7 @@ __global__ __launch_bounds__(256) void dh_reduce_kernel(const float* __restrict_
 #pragma unroll
       for (int c = 0; c < 8; ++c) s[c] *= a;
     }
-    store_n<bf16, 8>(dH + (int64_t)order[r] * H + n, s);
+    store_n<bf16, 8>(dH + (int64_t)live.token(r) * H + n, s);
   }
 }
 
@@ -1086,9 +1087,9 @@ struct GradWs {
   float *pmax, *psum;                // [T, nblk]
   float *zy, *loss_row, *valid_row;  // [N]
   float *shift, *alpha;              // [T]
-  bf16* Hc;                          // [T, H]: the chunk's hidden rows
+  bf16* Hc;                          // [T, H]: the chunk's hidden rows (masked)
   bf16* Hs;                          // [T, H]: alpha-scaled hidden rows (dW)
-  int *order, *n_live;               // [N], [1]
+  int *order, *n_live;               // [N], [1] (masked)
   int* tile_flags;                   // [ceil(T / 256)]
   float* part;                       // dH split-K partials
   size_t part_bytes;
@@ -1156,7 +1157,10 @@ int fwd_grad_impl(const bf16* hidden, int64_t ldh, const bf16* weight, int64_t l
   const int nblk = (int)nblocks(V);                                // loss only: 64 columns
   const int nsb = (int)((V + kShiftBlock - 1) / kShiftBlock);       // one pass: 128 columns
   const bool grads = d_hidden || d_weight;
-  token_order_kernel<<<1, 1024, 0, st>>>(labels, N, ignore, masked, w.order, w.n_live, n_valid);
+  if (masked && grads)
+    token_order_kernel<<<1, 1024, 0, st>>>(labels, N, ignore, w.order, w.n_live, n_valid);
+  else
+    count_valid_kernel<<<1, 1024, 0, st>>>(labels, N, ignore, n_valid);
   ML_LAUNCH_CHECK();
   int rc;
   for (int t0 = 0; t0 < N; t0 += T) {
@@ -1164,7 +1168,11 @@ int fwd_grad_impl(const bf16* hidden, int64_t ldh, const bf16* weight, int64_t l
     const bf16* hc = hidden + (int64_t)t0 * ldh;
     const int64_t* lc = labels + t0;
     const unsigned row_blocks = (unsigned)((Tc + 3) / 4);
-    Segment seg{{grads ? w.Hc : hc, grads ? H : ldh}, {weight, ldw}, H};
+    // the chunk's rows: gathered in the tokens' order, or as they lie
+    const bool gather = masked && grads;
+    const bf16* rows = gather ? w.Hc : hc;
+    const int64_t ldr = gather ? H : ldh;
+    Segment seg{{rows, ldr}, {weight, ldw}, H};
     Problem pb;
     rc = make_problem<R4Cfg>(pb, Tc, V, 1, &seg, kKMajor, kKMajor, 0);
     if (rc) return rc;
@@ -1182,12 +1190,11 @@ int fwd_grad_impl(const bf16* hidden, int64_t ldh, const bf16* weight, int64_t l
       ML_LAUNCH_CHECK();
       continue;
     }
-    const LiveRows live{w.n_live, t0, Tc};
-    const int* order = w.order + t0;
-    // 1. gathered rows, row shifts (label logits) and cleared tile flags
-    shift_kernel<TB><<<row_blocks, 256, 0, st>>>(hidden, ldh, weight, ldw, bias, labels, order,
-                                                 live, V, H, w.Hc, w.zy + t0, w.shift,
-                                                 w.tile_flags, n_tile_flags(Tc));
+    const LiveRows live{masked ? w.n_live : nullptr, masked ? w.order + t0 : nullptr, t0, Tc};
+    // 1. gathered rows (masked), row shifts (label logits) and cleared tile flags
+    shift_kernel<TB><<<row_blocks, 256, 0, st>>>(
+        hidden, ldh, weight, ldw, bias, labels, live, V, H, masked ? w.Hc : nullptr, w.zy + t0,
+        w.shift, w.tile_flags, n_tile_flags(Tc));
     ML_LAUNCH_CHECK();
     // 2. logits, e = exp(z - c) in bf16, (max, sum e) partials (r4 engine),
     // 3. lse, loss terms, row factors, label entries, scaled hidden rows;
@@ -1205,12 +1212,12 @@ int fwd_grad_impl(const bf16* hidden, int64_t ldh, const bf16* weight, int64_t l
       bf16* hs = d_weight ? w.Hs : nullptr;
       if (pass == 0)
         finalize_kernel<false><<<row_blocks, 256, 0, st>>>(
-            w.pmax, w.psum, nsb, w.shift, w.zy + t0, labels, order, live, ignore, Tc, V, n_valid,
-            w.E, V, w.Hc, H, hs, w.alpha, w.tile_flags, lse, w.loss_row, w.valid_row);
+            w.pmax, w.psum, nsb, w.shift, w.zy + t0, labels, live, ignore, Tc, V, n_valid, w.E, V,
+            rows, ldr, H, hs, w.alpha, w.tile_flags, lse, w.loss_row, w.valid_row);
       else
         finalize_kernel<true><<<row_blocks, 256, 0, st>>>(
-            w.pmax, w.psum, nsb, w.shift, w.zy + t0, labels, order, live, ignore, Tc, V, n_valid,
-            w.E, V, w.Hc, H, hs, w.alpha, w.tile_flags, lse, w.loss_row, w.valid_row);
+            w.pmax, w.psum, nsb, w.shift, w.zy + t0, labels, live, ignore, Tc, V, n_valid, w.E, V,
+            rows, ldr, H, hs, w.alpha, w.tile_flags, lse, w.loss_row, w.valid_row);
       ML_LAUNCH_CHECK();
     }
     if (d_hidden) {  // 4. dH_c = diag(alpha) (E' W) (split-K over the vocabulary)
@@ -1226,8 +1233,7 @@ int fwd_grad_impl(const bf16* hidden, int64_t ldh, const bf16* weight, int64_t l
       ML_LAUNCH_CHECK();
       const int64_t vecs = (int64_t)Tc * (H / 8);
       const unsigned blocks = (unsigned)std::min<int64_t>((vecs + 255) / 256, 2048);
-      dh_reduce_kernel<<<dim3(blocks), 256, 0, st>>>(w.part, splits, live, order, Tc, H, w.alpha,
-                                                     d_hidden);
+      dh_reduce_kernel<<<dim3(blocks), 256, 0, st>>>(w.part, splits, live, Tc, H, w.alpha, d_hidden);
       ML_LAUNCH_CHECK();
     }
     if (d_weight) {  // 5. dW (+)= E'^T (diag(alpha) H_c)

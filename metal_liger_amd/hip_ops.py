@@ -788,11 +788,11 @@ def flce_fwd_grad(hidden, weight, labels, bias=None, ignore_index: int = -100,
     dh = torch.empty(N, H, dtype=torch.bfloat16, device=dev) if need_dhidden else None
     dw = torch.empty(V, H, dtype=torch.bfloat16, device=dev) if need_dweight else None
     T = int(token_chunk) if token_chunk else flce_token_chunk(N, V)
+    fn = "ml_flce_fwd_grad_masked" if masked else "ml_flce_fwd_grad"
     wsb = _hip.query("ml_flce_fwd_grad_workspace_bytes", N, V, H, T, 1 if need_dhidden else 0)
     ws = torch.empty(max(wsb, 16), dtype=torch.uint8, device=dev)
     call(
-        "ml_flce_fwd_grad_masked" if masked else "ml_flce_fwd_grad", ptr(hidden), hidden.stride(0) if N > 0 else H, ptr(weight),
-        weight.stride(0), ptr(bias), dtype_tag(bias, "bias") if bias is not None else 0, ptr(labels),
+        fn, ptr(hidden), hidden.stride(0) if N > 0 else H, ptr(weight), weight.stride(0), ptr(bias), dtype_tag(bias, "bias") if bias is not None else 0, ptr(labels),
         N, V, H, int(ignore_index), T, ptr(loss), ptr(lse), ptr(n_valid), ptr(dh), ptr(dw), ptr(ws),
         ws.numel(), stream_of(weight),
     )

@@ -85,3 +85,23 @@ def test_masked_recomputes_flagged_rows(big):
     rdh, rdw = ref.flce_backward(h, w, lab, rlse, mask, torch.tensor(1.0), None, 8192)
     assert abs(loss.item() - rl.item()) <= 1e-3 * abs(rl.item())
     assert rel_fro(dh, rdh) <= 2e-2 and rel_fro(dw, rdw) <= 2e-2
+
+
+@pytest.mark.parametrize("chunk", [None, 256])
+def test_unmasked_reads_strided_rows_in_place(chunk):
+    """Without the mask nothing is gathered: rows of a wider tensor, ignored
+    tokens among them (their lse is computed, their gradients are zero)."""
+    h, w, lab = _case(700, 500, seed=13)
+    wide = torch.full((700, 160), float("nan"), dtype=BF)
+    wide[:, 8:144] = h
+    d = wide.cuda()[:, 8:144]
+    assert d.stride(0) == 160
+    loss, lse, nv, dh, dw = hip_ops.flce_fwd_grad(d, w.cuda(), lab.cuda(), None, -100,
+                                                  token_chunk=chunk)
+    rl, rlse, mask = ref.flce_forward(h, w, lab, None, -100, 384)
+    rdh, rdw = ref.flce_backward(h, w, lab, rlse, mask, torch.tensor(1.0), None, 384)
+    assert nv.item() == 500
+    assert abs(loss.item() - rl.item()) <= 1e-3 * abs(rl.item())
+    assert rel_fro(lse, rlse) <= 1e-5
+    assert rel_fro(dh, rdh) <= 2e-2 and rel_fro(dw, rdw) <= 2e-2
+    assert not dh[(lab == -100).cuda()].any()
