@@ -1577,6 +1577,10 @@ static int flce_fwd_grad(bool masked, const void* hidden, int64_t ldh, const voi
   // dW is written as 16-byte row vectors; dH is scaled as 16-byte vectors later
   ML_CHECK((!d_hidden || aligned16(d_hidden)) && (!d_weight || aligned16(d_weight)),
            "flce: gradients must be 16-byte aligned");
+  // rows are read as 16-byte vectors (the masked form gathers them, so that no
+  // product sees the caller's hidden)
+  ML_CHECK(n_tokens == 0 || (aligned16(hidden) && ldh % 8 == 0 && aligned16(weight) && ldw % 8 == 0),
+           "flce: hidden and weight must be 16-byte aligned, with row strides in multiples of 8");
   ML_CHECK(token_chunk > 0 && token_chunk < (1LL << 31), "flce: token_chunk must be positive");
   hipStream_t st = (hipStream_t)stream;
   const int64_t H = hidden_size;
