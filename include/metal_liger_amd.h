@@ -357,8 +357,9 @@ int ml_flce_scale_grads_f32(const float* grad_loss, float* d_hidden, int64_t n_h
  * X A_stack^T from the forward. Outputs: dX bf16 [n_tokens, in];
  * dA fp32 [3 rank, in] (dA_q, dA_k, dA_v stacked); dB[i] fp32 [out, rank].
  * in_features, out_features and rank must be multiples of 8; dX is written
- * as 16-byte rows and must be 16-byte aligned. No gradient for the frozen
- * base weights, as in the reference.
+ * and the operands are read as 16-byte vectors and must be 16-byte aligned
+ * (refused otherwise; B and XA of rank 16 may have any alignment). No gradient
+ * for the frozen base weights, as in the reference.
  */
 size_t ml_lora_qkv_bwd_workspace_bytes(int64_t n_tokens, int64_t in_features,
                                        const int64_t* out_features, int64_t rank);
@@ -394,7 +395,8 @@ int ml_lora_linear_bwd(const void* X, int64_t n_tokens, int64_t in_features, con
  * intermediate], BG, BU [intermediate, rank], BD [hidden, rank]; scale = HOST
  * floats {s_G, s_U, s_D}. Outputs: dX bf16 [n, hidden]; fp32 dA_GU [2 rank,
  * hidden], dA_D [rank, intermediate], dB_G, dB_U [intermediate, rank], dB_D
- * [hidden, rank] (dX 16-byte aligned: it is written as 16-byte rows).
+ * [hidden, rank] (dX 16-byte aligned: it is written as 16-byte rows; the
+ * operands as in ml_lora_qkv_bwd, gate and up of any alignment).
  * dH = dY W_D + s_D (dY B_D) A_D is formed in bf16 and the SwiGLU backward
  * then runs over it in place.
  * h may be NULL: it is then silu(gate) * up rounded to bf16 exactly as

@@ -1219,6 +1219,16 @@ extern "C" int ml_lora_xa(const void* X, int64_t n_tokens, int64_t in_features, 
   return ML_OK;
 }
 
+// Operands that the backward reads as 16-byte vectors, or straight into LDS, by
+// kernels that have no other path: aligned, and so refused otherwise before
+// anything is launched. At rank 16 the rank-r operands (B, X A^T) are read in
+// single elements and dwords; the products of other ranks share one rule.
+static bool all_aligned16(std::initializer_list<const void*> ptrs) {
+  for (const void* p : ptrs)
+    if (!aligned16(p)) return false;
+  return true;
+}
+
 // ------------------------------------------------------------------- QKV --
 
 static size_t qkv_partial_bytes(int64_t N, int64_t in_f, const int64_t* out_f, int nadp,
@@ -1264,7 +1274,11 @@ static int adapters_bwd(const char* what, int nadp, const void* X, int64_t n_tok
     ML_CHECK(dY[i] && W[i] && B[i] && dB[i], "%s: null pointer for adapter %d", what, i);
     ML_CHECK(out_features[i] > 0 && out_features[i] % 8 == 0 && out_features[i] < (1LL << 31),
              "%s: out_features[%d] must be a positive multiple of 8", what, i);
+    ML_CHECK(aligned16(dY[i]) && (rank == lora::kDyRank || aligned16(B[i])),
+             "%s: dY and B of adapter %d must be 16-byte aligned", what, i);
   }
+  ML_CHECK(aligned16(X) && (rank == lora::kDyRank || aligned16(XA)),
+           "%s: X and XA must be 16-byte aligned", what);
   const size_t need = adapters_bwd_ws_bytes(n_tokens, in_features, out_features, nadp, rank);
   ML_CHECK(aligned16(dX), "%s: dX must be 16-byte aligned (it is written as 16-byte rows)",
            what);
@@ -1412,6 +1426,9 @@ extern "C" int ml_lora_mlp_bwd(const void* X, int64_t n_tokens, int64_t hidden,
                XA_GU && hA_D && dX && dA_GU && dA_D && dB_G && dB_U && dB_D,
            "lora mlp: null pointer");
   ML_CHECK(aligned16(dX), "lora mlp: dX must be 16-byte aligned (it is written as 16-byte rows)");
+  ML_CHECK(all_aligned16({X, dY, h}) &&
+               (rank == lora::kDyRank || all_aligned16({BG, BU, BD, XA_GU, hA_D})),
+           "lora mlp: X, dY, h and the rank-r operands must be 16-byte aligned");
   const size_t need = ml_lora_mlp_bwd_workspace_bytes(n_tokens, hidden, intermediate, rank);
   ML_CHECK(workspace && workspace_bytes >= need, "lora mlp: workspace too small (%zu < %zu)",
            workspace_bytes, need);
