@@ -55,6 +55,18 @@ class _RepeatKV(torch.autograd.Function):
         return dk, dv, None
 
 
+def _plain_eager() -> bool:
+    """No torch.compile, functorch transform or forward-mode AD is at work. (The
+    latter two can only be told by private names; a torch without them counts as
+    not plain.)"""
+    try:
+        return not (torch.compiler.is_compiling()
+                    or torch._C._are_functorch_transforms_active()
+                    or forward_ad._current_level >= 0)
+    except AttributeError:
+        return False
+
+
 def _repeat_kv(key: torch.Tensor, value: torch.Tensor, groups: int):
     """key and value with their heads repeated: by the kernels for plain GPU
     tensors in eager mode, else (other devices and dtypes, ragged head sizes,
@@ -67,9 +79,7 @@ def _repeat_kv(key: torch.Tensor, value: torch.Tensor, groups: int):
             and key.dim() == 4 and key.shape[:3] == value.shape[:3]
             and key.shape[3] % row == 0 and value.shape[3] % row == 0
             and key.numel() > 0 and value.numel() > 0
-            and not torch.compiler.is_compiling()
-            and not torch._C._are_functorch_transforms_active()
-            and forward_ad._current_level < 0):
+            and _plain_eager()):
         return _RepeatKV.apply(key, value, groups)
     return _repeat_heads(key, groups), _repeat_heads(value, groups)
 
