@@ -430,7 +430,7 @@ def bench_lora_bwd(dev, timer, reps=20):
     hmid = hip_ops.swiglu_fwd(gate, up)
     ha_d = hip_ops.lora_xa(hmid, a_d)
 
-    def qkv():
+    def qkv():  # the Function's call without the launch that casts the adapters' gradients
         hip_ops.lora_qkv_bwd(x, dqkv, Wqkv, a_qkv, Bqkv, [s, s, s], xa, r)
 
     def mlp():  # h recomputed from gate and up, as the autograd path calls it

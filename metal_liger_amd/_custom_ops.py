@@ -375,6 +375,8 @@ def _(x2, w, xa, sb):
     return x2.new_empty((x2.shape[0], w.shape[0]), dtype=torch.bfloat16)
 
 
+# lora_qkv_out and lora_qkv_bwd (below): the QKV block on operands formed
+# beforehand; the Function calls lora_qkv_fwd and lora_qkv_bwd_packed.
 @torch.library.custom_op(f"{NS}::lora_qkv_out", mutates_args=(), device_types=_DEV)
 def lora_qkv_out(x2: Tensor, ws: List[Tensor], xa: Tensor, sbs: List[Tensor]) -> List[Tensor]:
     return hip_ops.lora_qkv_out(x2, ws, xa, sbs)

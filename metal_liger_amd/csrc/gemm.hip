@@ -231,12 +231,19 @@ extern "C" int ml_gemm_bf16_splitk(int64_t M, int64_t N, int64_t K, const void* 
   ML_CHECK(ksplit >= 1, "gemm: ksplit must be >= 1");
   gemm::Segment s{{static_cast<const bf16*>(A), lda}, {static_cast<const bf16*>(B), ldb}, (int)K};
   hipStream_t st = (hipStream_t)stream;
+  auto go = [&](auto fn) {
+    return fn(M, N, s, a_layout, b_layout, ksplit, C, ldc, c_dtype, alpha, beta, workspace,
+              workspace_bytes, st);
+  };
   switch (tile_cfg) {
-    case 0: return gemm::run_splitk<gemm::BigCfg>(M, N, s, a_layout, b_layout, ksplit, C, ldc, c_dtype, alpha, beta, workspace, workspace_bytes, st);
-    case 1: return gemm::run_splitk<gemm::TallCfg>(M, N, s, a_layout, b_layout, ksplit, C, ldc, c_dtype, alpha, beta, workspace, workspace_bytes, st);
-    case 2: return gemm::run_splitk<gemm::WideCfg>(M, N, s, a_layout, b_layout, ksplit, C, ldc, c_dtype, alpha, beta, workspace, workspace_bytes, st);
-    case 3: return gemm::run_splitk_r4<gemm::R4SCfg>(M, N, s, a_layout, b_layout, ksplit, C, ldc, c_dtype, alpha, beta, workspace, workspace_bytes, st);
-    case 4: return gemm::run_splitk_r4<gemm::R4Cfg>(M, N, s, a_layout, b_layout, ksplit, C, ldc, c_dtype, alpha, beta, workspace, workspace_bytes, st);
-    default: set_error("gemm: tile_cfg must be 0 (256x256), 1 (256x32), 2 (64x256), 3 (128x128) or 4 (256x256, K-major A)"); return ML_ERR_INVALID;
+    case 0: return go(gemm::run_splitk<gemm::BigCfg>);
+    case 1: return go(gemm::run_splitk<gemm::TallCfg>);
+    case 2: return go(gemm::run_splitk<gemm::WideCfg>);
+    case 3: return go(gemm::run_splitk_r4<gemm::R4SCfg>);
+    case 4: return go(gemm::run_splitk_r4<gemm::R4Cfg>);
+    default:
+      set_error("gemm: tile_cfg must be 0 (256x256), 1 (256x32), 2 (64x256), 3 (128x128) or 4 "
+                "(256x256, K-major A)");
+      return ML_ERR_INVALID;
   }
 }

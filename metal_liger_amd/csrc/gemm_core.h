@@ -1788,16 +1788,14 @@ struct EpiPartial {
   }
 };
 
-// out[m, n] = alpha * row_scale[m] * sum_s P[s][m][n] + beta * out[m, n]
-// (fixed order; row_scale null: 1). Four consecutive elements per thread when
-// N % 4 == 0 (16-byte partial loads, the splits unrolled so several loads are
-// in flight), one otherwise.
+// out[m, n] = alpha * sum_s P[s][m][n] + beta * out[m, n] (fixed order). Four
+// consecutive elements per thread when N % 4 == 0 (16-byte partial loads, the
+// splits unrolled so several loads are in flight), one otherwise.
 template <typename TC>
 __global__ __launch_bounds__(256) void reduce_partials_kernel(const float* __restrict__ P,
                                                               int ksplit, int M, int N,
                                                               TC* __restrict__ out, int64_t ldo,
-                                                              float alpha, float beta,
-                                                              const float* __restrict__ row_scale = nullptr) {
+                                                              float alpha, float beta) {
   const int64_t total = (int64_t)M * N;
   if (N % 4 == 0) {
     const int64_t nv = total / 4;
@@ -1825,15 +1823,14 @@ __global__ __launch_bounds__(256) void reduce_partials_kernel(const float* __res
       }
       const int64_t m = e / N, n = e - m * N;
       TC* p = out + m * ldo + n;
-      const float a = row_scale ? alpha * row_scale[m] : alpha;
       if (vec) {
-        const float r[4] = {a * s[0], a * s[1], a * s[2], a * s[3]};
+        const float r[4] = {alpha * s[0], alpha * s[1], alpha * s[2], alpha * s[3]};
         store_n<TC, 4>(p, r);
         continue;
       }
 #pragma unroll
       for (int c = 0; c < 4; ++c) {
-        float r = a * s[c];
+        float r = alpha * s[c];
         if (beta != 0.f) r += beta * to_f32(p[c]);
         p[c] = from_f32<TC>(r);
       }
@@ -1846,7 +1843,7 @@ __global__ __launch_bounds__(256) void reduce_partials_kernel(const float* __res
     for (int k = 0; k < ksplit; ++k) s += P[(int64_t)k * total + e];
     const int64_t m = e / N, n = e - m * N;
     TC* p = out + m * ldo + n;
-    float r = (row_scale ? alpha * row_scale[m] : alpha) * s;
+    float r = alpha * s;
     if (beta != 0.f) r += beta * to_f32(*p);
     *p = from_f32<TC>(r);
   }
@@ -1967,7 +1964,7 @@ inline int launch_store_group(const Problem* pbs, int count, int lb, void* const
 // then out = alpha * sum + beta * out.
 template <class C, int LA, int LB, typename TC>
 inline int launch_splitk(const Problem& pb, float* ws, TC* out, int64_t ldo, float alpha, float beta,
-                         hipStream_t st, const float* row_scale = nullptr) {
+                         hipStream_t st) {
   EpiPartial epi{ws, pb.M, pb.N};
   gemm_kernel<C, LA, LB, EpiPartial><<<dim3(grid_blocks(pb)), C::THREADS, 0, st>>>(pb, epi);
   ML_LAUNCH_CHECK();
@@ -1976,8 +1973,7 @@ inline int launch_splitk(const Problem& pb, float* ws, TC* out, int64_t ldo, flo
   int64_t blocks = (total / per_thread + 255) / 256;
   blocks = blocks < 2048 ? (blocks > 0 ? blocks : 1) : 2048;
   reduce_partials_kernel<TC><<<dim3((unsigned)blocks), 256, 0, st>>>(ws, pb.ksplit, pb.M, pb.N,
-                                                                     out, ldo, alpha, beta,
-                                                                     row_scale);
+                                                                     out, ldo, alpha, beta);
   ML_LAUNCH_CHECK();
   return ML_OK;
 }

@@ -11,14 +11,15 @@
 //   dA  = P^T X                [r, in]       one pass over X (ptx_pass_kernel),
 //                              else 64x256 tiles, split-K over tokens
 //   dX  = [dY_1 | .. | dY_n | P_1..n] [W_1; ..; W_n; A_1..n]
-//         ONE 256x256-tile GEMM over the K-concatenation of every adapter's
-//         dY with its W plus the stacked rank-r terms (K = sum(out) + n r).
+//         ONE GEMM over the K-concatenation of every adapter's dY with its W
+//         plus the stacked rank-r terms (K = sum(out) + n r), on the tile and
+//         split that run_product picks.
 // The MLP backward first forms dH = dY_D W_D + P_D A_D (bf16), runs the
 // SwiGLU backward over it in place (sigmoid recomputed), then treats
 // (d_gate, d_up) as the output grads of the gate / up adapters; at rank 16
 // one pass (mlp_mid_kernel) does the SwiGLU backward, the gate / up dY-pass
-// work and P_D^T h. Partials are
-// summed in a fixed order, so every gradient is bit-reproducible.
+// work and P_D^T h. Partials are summed in a fixed order, so every gradient is
+// bit-reproducible.
 #include <algorithm>
 
 #include "gemm_core.h"
@@ -1016,13 +1017,13 @@ __global__ __launch_bounds__(256) void unpack_kernel(const UnpackArgs args) {
 // products (F.linear(x, A) of ops/fused_lora.py:79-81). A workgroup of 8
 // waves owns 16 MT rows of X (MT = 2; 1 where that leaves CUs without work: a
 // wave's chain of loads is what such a launch waits for); wave w takes the w-th
-// eighth of the k range in steps of 32, with the MFMA
-// operands loaded straight from global memory in their register layout
-// (lane l: 16 bytes of row l % 16 at k offset 8 (l / 16)), and the
-// waves' [32, 16 NT] fp32 sums meet in LDS in a fixed order before the bf16
-// store. X is read once from HBM, A (<= 256 KB) from L2; no split-K partials
-// and no second launch. Rows past N and columns past R are not stored;
-// lanes whose k lies past K contribute zeros (K % 8 == 0).
+// eighth of the k range in steps of 32, with the MFMA operands loaded straight
+// from global memory in their register layout (lane l: 16 bytes of row l % 16 at
+// k offset 8 (l / 16)), and the waves' [16 MT, 16 NT] fp32 sums meet in LDS in a
+// fixed order before the bf16 store. X is read once per blockIdx.y (up to 64 of
+// A's rows), A (2 R K bytes, 768 KB for 64 rows of 6144) by every workgroup, from
+// L2; no split-K partials and no second launch. Rows past N and columns past R
+// are not stored; lanes whose k lies past K contribute zeros (K % 8 == 0).
 constexpr int kXaWaves = 8;
 
 template <int NT, int MT>
@@ -1251,8 +1252,9 @@ static size_t qkv_partial_bytes(int64_t N, int64_t in_f, const int64_t* out_f, i
 }
 
 // Backward of nadp (1..3) adapters that share the input X: P_i and dB_i by
-// one pass over each dY_i (rank 16) or split-K skinny products, dA = P^T X,
-// and dX = [dY_1 | ... | P] [W_1; ...; A_stack] as one K-concatenated GEMM.
+// one pass over each dY_i (ranks 16, 32, 48 and 64) or split-K skinny products,
+// dA = P^T X, and dX = [dY_1 | ... | P] [W_1; ...; A_stack] as one
+// K-concatenated GEMM.
 static size_t adapters_bwd_ws_bytes(int64_t N, int64_t IN, const int64_t* out_f, int nadp,
                                     int64_t r) {
   return lora::align256((size_t)(N * nadp * r) * 2) + qkv_partial_bytes(N, IN, out_f, nadp, r);

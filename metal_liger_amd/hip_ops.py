@@ -792,9 +792,10 @@ def flce_fwd_grad(hidden, weight, labels, bias=None, ignore_index: int = -100,
     wsb = _hip.query("ml_flce_fwd_grad_workspace_bytes", N, V, H, T, 1 if need_dhidden else 0)
     ws = torch.empty(max(wsb, 16), dtype=torch.uint8, device=dev)
     call(
-        fn, ptr(hidden), hidden.stride(0) if N > 0 else H, ptr(weight), weight.stride(0), ptr(bias), dtype_tag(bias, "bias") if bias is not None else 0, ptr(labels),
-        N, V, H, int(ignore_index), T, ptr(loss), ptr(lse), ptr(n_valid), ptr(dh), ptr(dw), ptr(ws),
-        ws.numel(), stream_of(weight),
+        fn, ptr(hidden), hidden.stride(0) if N > 0 else H, ptr(weight), weight.stride(0), ptr(bias),
+        dtype_tag(bias, "bias") if bias is not None else 0, ptr(labels), N, V, H, int(ignore_index),
+        T, ptr(loss), ptr(lse), ptr(n_valid), ptr(dh), ptr(dw), ptr(ws), ws.numel(),
+        stream_of(weight),
     )
     return loss, lse, n_valid, _flce_unpad(dh, N, H0), _flce_unpad(dw, V0, H0)
 

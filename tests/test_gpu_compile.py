@@ -79,9 +79,10 @@ def test_opcheck_flce_ops(dev):
     w = _bf((V, H), 21, dev, 0.05)
     lab = torch.randint(0, V, (N,), generator=torch.Generator().manual_seed(22)).to(dev)
     lab[::7] = -100
-    for need_h, need_w in ((True, True), (True, False)):
-        torch.library.opcheck(ops.flce_fwd_grad.default, (h, w, lab, None, -100, need_h, need_w),
-                              test_utils=CHECKS)
+    for op in (ops.flce_fwd_grad, ops.flce_fwd_grad_masked):   # the latter is the loss's
+        for need_h, need_w in ((True, True), (True, False)):
+            torch.library.opcheck(op.default, (h, w, lab, None, -100, need_h, need_w),
+                                  test_utils=CHECKS)
     loss, lse, n_valid, dh, dw = ops.flce_fwd_grad(h, w, lab, None, -100, True, True)
     g = torch.full((), 0.5, device=dev)
     torch.library.opcheck(ops.flce_scale_grads.default, (g, dh.clone(), dw.clone()),

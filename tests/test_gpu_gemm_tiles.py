@@ -31,6 +31,28 @@ def test_tiles(m, n, k, ksplit, tile_cfg):
                    ref, k)
 
 
+@pytest.mark.parametrize("tile_cfg", [3, 4])
+@pytest.mark.parametrize("ksplit", [1, 3])
+@pytest.mark.parametrize("m,n,k", [(127, 136, 200), (257, 264, 1000)])
+def test_tiles_add_to_c(m, n, k, ksplit, tile_cfg):
+    """alpha A B + beta C, in every store of the tiles and of the split's
+    reduction, at an N that no tile divides; columns past N stay."""
+    g = torch.Generator().manual_seed(m + k)
+    a = torch.randn(m, k, generator=g).bfloat16().cuda()
+    b = torch.randn(n, k, generator=g).bfloat16().cuda()
+    for dt in (torch.float32, torch.bfloat16):
+        wide = torch.randn(m, n + 8, generator=g).to(dt).cuda()
+        c = wide[:, :n]
+        ref = 0.5 * (a.double() @ b.double().t()) - 1.5 * c.double()
+        rest = wide[:, n:].clone()
+        hip_ops.matmul(a, b, b_t=True, out=c, alpha=0.5, beta=-1.5, tile_cfg=tile_cfg,
+                       ksplit=ksplit)
+        # the product's error bound, and C's own share: exact in the products,
+        # one more rounding of the sum (fp32) or the same one (bf16)
+        _check(c, ref, k)
+        assert torch.equal(wide[:, n:], rest)
+
+
 @pytest.mark.parametrize("b_layout", [0, 1])
 @pytest.mark.parametrize("m,n,ks", [(16, 1024, (2048, 8)), (200, 2048, (1000, 72, 3000, 24)),
                                     (513, 136, (72, 4104)), (1, 8, (64, 64))])
