@@ -244,7 +244,7 @@ def floats(vals) -> ctypes.Array:
 
 def stream_of(t: torch.Tensor) -> int:
     # the raw handle of torch.cuda.current_stream(t.device), without the Stream
-    # object (0.1 against 2.0 us per launch) where this torch has the private call
+    # object (0.2 against 2.0 us per launch) where this torch has the private call
     # for it; that would take a CPU tensor's device index for the current GPU
     if not t.is_cuda:
         ensure_rocm_device(t)

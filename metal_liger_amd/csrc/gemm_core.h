@@ -1992,10 +1992,11 @@ inline size_t splitk_ws_bytes(const Problem& pb) {
 // [2064, 6144]: 270 against 205 us).
 // product_us estimates a launch of `items` work items of kt 64-wide k-tiles
 // from measurements at M = 16 .. 8192, N = 1024 .. 6144, K = 512 .. 12352 on
-// one MI355X (the choice it makes was 2% slower than the best of the
-// measured ones on average, 20% at most): whole rounds of one workgroup per
-// CU (256) or two (128), then a partly filled round, whose k-tiles run
-// faster the emptier the chip is.
+// one MI355X (profiles/gemm_tile_sweep.md: the choice it makes was 1.8% slower
+// than the best of the measured ones on average, 19% at most; the constants
+// hold for its 256 CUs): whole rounds of one workgroup per CU (256) or two
+// (128), then a partly filled round, whose k-tiles run faster the emptier the
+// chip is.
 inline double product_us(int tile, int64_t items, int kt) {
   if (tile == 256) {
     const int64_t full = items / 256, rem = items % 256;
